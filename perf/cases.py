@@ -35,8 +35,9 @@ from motioncor3_amd import lib as L
 from motioncor3_amd.synth import MovieRecipe, eer_stream_7bit
 
 # frame sizes of cameras in use (counting and super-resolution modes, and a
-# movie whose frames are stored turned by 90 degrees)
-FRAMES = [(3838, 3710), (4096, 4096), (5760, 4092), (4092, 5760), (7676, 7420), (8192, 8192)]
+# movie whose frames are stored turned by 90 degrees; 5760 rows are not a
+# supported height)
+FRAMES = [(3838, 3710), (4096, 4096), (5760, 4092), (3710, 3838), (7676, 7420), (8192, 8192)]
 # the patch sizes of movies with a 2048-row alignment size
 GRIDS = [(5, 5), (7, 5), (6, 4), (3, 3)]
 
@@ -91,7 +92,7 @@ def _length(rng, lo, hi, step=1):
         for f in range(2, 152):
             while m % f == 0:
                 m //= f
-        if m == 1:
+        if m == 1 and n != 5760:
             return n
 
 
