@@ -12,6 +12,7 @@
 #include <string>
 #include <vector>
 #include "mc_common.h"
+#include "mc_fft_gp.h"
 #include "mc_spec.h"
 
 // Tile shape of the two passes: C = the largest power of two <= MC_TILE_CMAX
@@ -33,6 +34,7 @@ struct Fft2D {
     int cx = 0;                // W/2 + 1
     int C = 0;                 // column block of the T layout
     int R = 0;                 // rows per row-pass workgroup
+    int Cc = 0;                // columns per workgroup of the correlation's stage kernel
     FftPlan1 row{}, col{};
     cfloat* post_tw = nullptr; // m+1 entries e^{-2 pi i k / W}
     cfloat* row_tw = nullptr;  // owned device tables
@@ -48,6 +50,9 @@ struct Fft2D {
     int row_var = 0, col_var = 0;
     // the same for the inverse passes (C2R rows, inverse columns)
     int row_var_inv = 0, col_var_inv = 0;
+    // run-time radix passes of a side without compiled kernels (n 0: none)
+    GpPlan row_gp{}, col_gp{};
+    GpTables row_gt, col_gt;
 };
 
 // Per-transform phase factors e^{i(kx*ax + ky*ay)} applied on load (skip

@@ -11,74 +11,11 @@
 #include <vector>
 
 #include "mc_fft.h"
+#include "mc_fft_args.h"
 #include "mc_fft_ct.h"
 #include "mc_fft_rp.h"
 
 namespace {
-
-struct RowR2CArgs {
-    FftPlan1 plan;
-    int H, m, C, R;
-    const float* in;
-    long long pitch, in_bstride;
-    int in_mod;            // transform b reads image b % in_mod (0: b)
-    const int* win;        // (x0, y0) per b / in_mod, or null
-    cfloat* T;
-    long long t_bstride;
-    const cfloat* post_tw;
-    float scale;
-    float* dc;             // |row DC| per (transform, row) of the output, or null
-};
-
-struct RowC2RArgs {
-    FftPlan1 plan;
-    int H, m, C, R;
-    const cfloat* T;
-    long long t_bstride;
-    float* out;
-    long long pitch, out_bstride;
-    const cfloat* post_tw;
-    int clamp;
-};
-
-struct ColFwdArgs {
-    FftPlan1 plan;
-    int H, ncols, C;
-    const cfloat* T;
-    long long t_bstride;
-    cfloat* S;
-    long long s_bstride;
-    cfloat* X;
-    int xcx, xcy;
-    long long x_bstride;
-    const float* s_g;      // store factors of a reduced S format (per transform)
-    const float* x_g;      // store factors of a reduced X format
-};
-
-struct ColInvArgs {
-    FftPlan1 plan;
-    int H, ncols, C;
-    const cfloat* S;
-    long long s_bstride;
-    int src_cx, src_cy;
-    const cfloat* phA;
-    const cfloat* phB;
-    cfloat* T;
-    long long t_bstride;
-    const float* s_inv;    // load factors of a reduced S format (per transform)
-};
-
-// Util/GFourierResize2D.cu:15-35 row map: output row yo of a spectrum with
-// `outy` rows taken from a spectrum with `iny` rows, -1 if unmapped.
-__device__ __forceinline__ int resize_row(int yo, int outy, int iny) {
-    int y = yo;
-    if (y > outy / 2) {
-        y -= outy;
-        if (y <= -iny / 2) return -1;
-        return y + iny;
-    }
-    return (y > iny / 2) ? -1 : y;
-}
 
 #define MC_IO_UNROLL 8
 
@@ -599,14 +536,6 @@ __global__ __launch_bounds__(NT) void k_cols_inv_ct(ColInvArgs a) {
 // workgroup held unpadded in LDS (C*H*8 bytes).  Forward: staging T -> S
 // (+ the xcf crop X); inverse: S (phase factors, conjugated) -> T.  Same
 // results as the stage-by-stage kernels up to FP32 rounding order.
-
-// Output row of a cropped (xcy-row) spectrum that input row y maps to, or -1
-// (the inverse of resize_row for xcy < H).
-__device__ __forceinline__ int crop_row(int y, int xcy, int H) {
-    if (y <= xcy / 2) return y;
-    const int d = H - xcy;
-    return (y > xcy / 2 + d) ? y - d : -1;
-}
 
 template <int H, int CW, int NT, int FS, int FX, int SC>
 __global__ __launch_bounds__(NT) void k_cols_fwd_rp(ColFwdArgs a, const cfloat* __restrict__ ptw) {
@@ -1168,7 +1097,7 @@ hipError_t mc_launch_spec_scale(const float* dc, int rows, int batch, float* g, 
 }
 
 int mc_fft_init_constants() {
-    if (mc_upload_prime_table() != 0) return -1;
+    if (mc_upload_prime_table() != 0 || mc_fft_gp_init() != 0) return -1;
     if (!g_attr_done) {
         set_lds_attr(k_rows_r2c);
         set_lds_attr(k_rows_c2r);
@@ -1198,6 +1127,19 @@ int mc_fft2d_create(Fft2D* p, int W, int H) {
     // Heights with a register-pass column schedule read a few columns of a
     // wider staging chunk, so the row passes move whole 128-byte lines.
     if (rp_has(H) && H >= 1024) C = MC_TILE_CT;
+    p->Cc = C;
+    // Columns without a compiled kernel run the run-time radix passes, which
+    // take as many of a chunk's columns as LDS holds: at least MC_TILE_CT
+    // columns per chunk, so that the row passes move whole 32-byte sectors.
+    // (Heights whose chunk exceeds the stage kernels' LDS stay unsupported.)
+    bool compiled = (long long)C * H > MC_LDS_ELEMS;
+#define X(HH, CC, NT, SC) compiled = compiled || (H == HH && C % CC == 0);
+    MC_RP_COL_SPECS(X)
+#undef X
+#define X(HH, CC, NT) compiled = compiled || (H == HH && C == CC);
+    MC_COL_SPECS(X)
+#undef X
+    if (!compiled && gp_plan(H, &p->col_gp, &p->col_gt)) C = std::max(C, MC_TILE_CT);
     p->C = C;
     int R = 1;
     const int want = std::max((MC_TILE_RC + C - 1) / C, 2);
@@ -1210,6 +1152,14 @@ int mc_fft2d_create(Fft2D* p, int W, int H) {
     while (R * 2 <= rmax && (R * 2) * per_row <= budget) R *= 2;
     if (R * per_row > MC_LDS_ELEMS) return -1;
     p->R = R;
+    compiled = false;
+#define X(MM, RRR, CCC, NT, SC) compiled = compiled || (m == MM && C == CCC);
+    MC_RP_ROW_SPECS(X)
+#undef X
+#define X(MM, RRR, CCC) compiled = compiled || (m == MM && R == RRR && C == CCC);
+    MC_ROW_SPECS(X)
+#undef X
+    if (!compiled) gp_plan(m, &p->row_gp, &p->row_gt);
     if (build_plan1(&p->row, &p->row_tw, m) != 0) return -2;
     if (build_plan1(&p->col, &p->col_tw, H) != 0) return -2;
     std::vector<cfloat> pt(m + 1);
@@ -1242,6 +1192,8 @@ void mc_fft2d_destroy(Fft2D* p) {
     if (p->row_tw) (void)hipFree(p->row_tw);
     if (p->col_tw) (void)hipFree(p->col_tw);
     if (p->post_tw) (void)hipFree(p->post_tw);
+    gp_free(&p->row_gt);
+    gp_free(&p->col_gt);
     for (cfloat* t : {p->col_ptw, p->row_ptw, p->col_ptw1, p->row_ptw1})
         if (t) (void)hipFree(t);
     p->row_tw = p->col_tw = p->post_tw = p->col_ptw = p->row_ptw = p->col_ptw1 = p->row_ptw1 = nullptr;
@@ -1346,6 +1298,7 @@ hipError_t mc_rows_r2c_mod(const Fft2D& p, const float* in, long long pitch, lon
     }
     MC_ROW_SPECS(X)
 #undef X
+    if (p.row_gp.n) return gp_rows_r2c(p.row_gp, a, batch, s);
     hipLaunchKernelGGL(k_rows_r2c, grid, dim3(MC_NTHR), lds, s, a);
     return hipGetLastError();
 }
@@ -1388,6 +1341,7 @@ hipError_t mc_rows_c2r(const Fft2D& p, const cfloat* T, long long t_bstride, flo
     }
     MC_ROW_SPECS(X)
 #undef X
+    if (p.row_gp.n) return gp_rows_c2r(p.row_gp, a, batch, s);
     hipLaunchKernelGGL(k_rows_c2r, grid, dim3(MC_NTHR), lds, s, a);
     return hipGetLastError();
 }
@@ -1427,6 +1381,7 @@ hipError_t mc_cols_fwd(const Fft2D& p, const cfloat* T, long long t_bstride, cfl
     }
     MC_COL_SPECS(X)
 #undef X
+    if (p.col_gp.n) return gp_cols_fwd(p.col_gp, a, batch, s);
     if ((long long)p.C * p.H > MC_LDS_ELEMS) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(k_cols_fwd, grid, dim3(MC_NTHR), lds, s, a);
     return hipGetLastError();
@@ -1465,6 +1420,7 @@ hipError_t mc_cols_inv(const Fft2D& p, const cfloat* S, long long s_bstride, int
     }
     MC_COL_SPECS(X)
 #undef X
+    if (p.col_gp.n) return gp_cols_inv(p.col_gp, a, batch, s);
     if ((long long)p.C * p.H > MC_LDS_ELEMS) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(k_cols_inv, grid, dim3(MC_NTHR), lds, s, a);
     return hipGetLastError();

@@ -17,38 +17,6 @@ __host__ __device__ constexpr int ct_spf(int n) {
         if (n % p == 0) return p;
     return n;
 }
-// ---- compile-time trigonometry (Taylor series in double, |x| <= pi) ----
-__host__ __device__ constexpr double rp_pi() { return 3.14159265358979323846; }
-__host__ __device__ constexpr double rp_sin_red(double x) {
-    double term = x, sum = x;
-    for (int n = 1; n < 30; n++) {
-        term *= -x * x / ((2.0 * n) * (2.0 * n + 1.0));
-        sum += term;
-    }
-    return sum;
-}
-__host__ __device__ constexpr double rp_cos_red(double x) {
-    double term = 1.0, sum = 1.0;
-    for (int n = 1; n < 30; n++) {
-        term *= -x * x / ((2.0 * n - 1.0) * (2.0 * n));
-        sum += term;
-    }
-    return sum;
-}
-// cos and sin of 2 pi a / b for integers, argument reduced to [-pi, pi]
-__host__ __device__ constexpr double rp_cos2pi(int a, int b) {
-    int r = a % b;
-    if (r < 0) r += b;
-    if (2 * r > b) r -= b;
-    return rp_cos_red(2.0 * rp_pi() * r / b);
-}
-__host__ __device__ constexpr double rp_sin2pi(int a, int b) {
-    int r = a % b;
-    if (r < 0) r += b;
-    if (2 * r > b) r -= b;
-    return rp_sin_red(2.0 * rp_pi() * r / b);
-}
-
 // ---- composite register DFT: v[k] = sum_t v[t] e^{-2 pi i t k / R} ----
 __host__ __device__ constexpr int rp_first(int r) {
     // leading factor of a composite register DFT: 4 or 2 for even sizes

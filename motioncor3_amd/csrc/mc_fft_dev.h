@@ -11,6 +11,38 @@
 #pragma once
 #include "mc_common.h"
 
+// ---- compile-time trigonometry (Taylor series in double, |x| <= pi) ----
+__host__ __device__ constexpr double rp_pi() { return 3.14159265358979323846; }
+__host__ __device__ constexpr double rp_sin_red(double x) {
+    double term = x, sum = x;
+    for (int n = 1; n < 30; n++) {
+        term *= -x * x / ((2.0 * n) * (2.0 * n + 1.0));
+        sum += term;
+    }
+    return sum;
+}
+__host__ __device__ constexpr double rp_cos_red(double x) {
+    double term = 1.0, sum = 1.0;
+    for (int n = 1; n < 30; n++) {
+        term *= -x * x / ((2.0 * n - 1.0) * (2.0 * n));
+        sum += term;
+    }
+    return sum;
+}
+// cos and sin of 2 pi a / b for integers, argument reduced to [-pi, pi]
+__host__ __device__ constexpr double rp_cos2pi(int a, int b) {
+    int r = a % b;
+    if (r < 0) r += b;
+    if (2 * r > b) r -= b;
+    return rp_cos_red(2.0 * rp_pi() * r / b);
+}
+__host__ __device__ constexpr double rp_sin2pi(int a, int b) {
+    int r = a % b;
+    if (r < 0) r += b;
+    if (2 * r > b) r -= b;
+    return rp_sin_red(2.0 * rp_pi() * r / b);
+}
+
 // cos/sin(2 pi j / P) for the register-butterfly primes, [cos..., sin...].
 #define MC_PRIMES_TABLE_LEN 320
 static __constant__ float g_pcs[MC_PRIMES_TABLE_LEN];
@@ -21,7 +53,7 @@ __host__ __device__ constexpr int mc_prime_off(int P) {
            P == 17 ? 78 : P == 19 ? 112 : P == 23 ? 150 : P == 29 ? 196 : P == 31 ? 254 : -1;
 }
 
-static int mc_upload_prime_table() {
+[[maybe_unused]] static int mc_upload_prime_table() {
     static const int primes[] = {3, 5, 7, 11, 13, 17, 19, 23, 29, 31};
     float h[MC_PRIMES_TABLE_LEN] = {0};
     for (int P : primes) {
@@ -35,11 +67,33 @@ static int mc_upload_prime_table() {
     return hipMemcpyToSymbol(HIP_SYMBOL(g_pcs), h, sizeof(h)) == hipSuccess ? 0 : -1;
 }
 
+#ifdef MC_PRIME_LITERALS
+// the same table as compile-time constants: the butterflies then take their
+// coefficients as instruction literals, not through scalar registers
+struct PrimeTab {
+    float c[32];
+    float s[32];
+};
+template <int P>
+__host__ __device__ constexpr PrimeTab prime_tab() {
+    PrimeTab t{};
+    for (int j = 0; j < P; j++) {
+        t.c[j] = (float)rp_cos2pi(j, P);
+        t.s[j] = (float)rp_sin2pi(j, P);
+    }
+    return t;
+}
+#endif
+
 // y[k] = sum_t x[t] e^{-2 pi i t k / P}, symmetric-pair form.
 template <int P>
 static __device__ __forceinline__ void bfly_prime(cfloat* v) {
     constexpr int H = (P - 1) / 2;
+#ifdef MC_PRIME_LITERALS
+    constexpr PrimeTab TAB = prime_tab<P>();
+#else
     constexpr int OFF = mc_prime_off(P);
+#endif
     cfloat u[H], w[H];
     const cfloat x0 = v[0];
     cfloat y0 = x0;
@@ -56,8 +110,12 @@ static __device__ __forceinline__ void bfly_prime(cfloat* v) {
 #pragma unroll
         for (int t = 1; t <= H; t++) {
             const int idx = (t * k) % P;
+#ifdef MC_PRIME_LITERALS
+            const float c = TAB.c[idx], s = TAB.s[idx];
+#else
             const float c = g_pcs[OFF + idx];
             const float s = g_pcs[OFF + P + idx];
+#endif
             ax = fmaf(u[t - 1].x, c, ax);
             ay = fmaf(u[t - 1].y, c, ay);
             bx = fmaf(w[t - 1].x, s, bx);
@@ -234,7 +292,7 @@ static __device__ __noinline__ void fft_stage_big(cfloat* lds, int n, int batch,
 }
 
 // Forward FFT of `batch` contiguous sequences of length P.n in LDS.
-static __device__ void fft_lds_fwd(cfloat* lds, int batch, const FftPlan1& P) {
+[[maybe_unused]] static __device__ void fft_lds_fwd(cfloat* lds, int batch, const FftPlan1& P) {
     for (int s = 0; s < P.nst; s++) {
         const FftStage st = P.st[s];
         switch (st.r) {

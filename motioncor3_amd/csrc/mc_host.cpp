@@ -718,7 +718,7 @@ int run_iterative_classes(mc_ctx* c, const char* tag, const IterClass* cls, int 
         }
         {
             KTimer kt(c, timed ? "correlate" : "");
-            if ((e = mc_launch_correlate(pl->col, pl->col_ptw, pl->C, nullptr, S, A, B, st, cx_max, H, b,
+            if ((e = mc_launch_correlate(pl->col, pl->col_ptw, pl->Cc, nullptr, S, A, B, st, cx_max, H, b,
                                          phase_only, seay, T1, s, f_fmt, nullptr)))
                 return e;
         }
@@ -775,7 +775,7 @@ int run_iterative_classes(mc_ctx* c, const char* tag, const IterClass* cls, int 
                      "%s|%d|%d|%d %d %d %d %d %d %d|%.9g %d %d %d %d|%p %p %p %p %p %p %p %p %p %p "
                      "%p %p %p %p %p %p %p %p %p %p %p %d %p|%d %p %p %d|",
                      tag, it0, it1, J, NT, H, max_iter, cx_max, G_max, tiles, (double)bft, phase_only,
-                     seax, seay, pl->C, (void*)A, (void*)B, (void*)S, (void*)T1, (void*)win,
+                     seax, seay, pl->Cc, (void*)A, (void*)B, (void*)S, (void*)T1, (void*)win,
                      (void*)st.tmp, (void*)st.total, (void*)st.gshift, (void*)st.final_,
                      (void*)st.errors, (void*)st.iters, (void*)st.done, (void*)st.gstart,
                      (void*)st.gsize, (void*)st.fgroup, (void*)st.gcent, (void*)st.fcent,
@@ -2338,7 +2338,7 @@ int mc_group_correlate_window(mc_ctx* c, const float* sum_spec, const float* grp
     MC_BUF(T1, cfloat, "api_T1", (size_t)sea_y * cx);
     MC_BUF(win, float, "api_win", (size_t)sea_x * sea_y);
     cfloat* twW = row_twiddles(c, W);
-    MC_TRY(mc_launch_correlate(pl->col, pl->col_ptw, pl->C, (const cfloat*)grp_spec, (const cfloat*)sum_spec, A,
+    MC_TRY(mc_launch_correlate(pl->col, pl->col_ptw, pl->Cc, (const cfloat*)grp_spec, (const cfloat*)sum_spec, A,
                                B, st, cx, H, bfactor, phase_only, sea_y, T1, c->stream));
     MC_TRY(mc_launch_row_dft(T1, twW, nullptr, 1, 1, cx, W, sea_x, sea_y, win, c->stream));
     MC_TRY(hipMemcpyAsync(window_host, win, sizeof(float) * sea_x * sea_y, hipMemcpyDeviceToHost,

@@ -195,3 +195,65 @@ def test_autotune_keeps_alignment_results():
                 assert np.linalg.norm(x - rep_o["sums"][i]) / np.linalg.norm(rep_o["sums"][i]) < 1e-4, i
     finally:
         c.close()
+
+
+# lengths without compiled kernels: one, two, three and four passes, the
+# largest radices, odd and even last radices, chirp convolutions from the
+# smallest (37) to the longest that fits LDS (8191)
+RUN_TIME_SIZES = [(4, 2), (10, 7), (12, 31), (66, 33), (74, 41), (146, 73), (128, 202), (682, 682), (1000, 600),
+                  (2838, 1919), (3838, 3710), (720, 2880), (64, 7105), (16382, 64), (64, 8191)]
+
+
+@pytest.mark.parametrize("W,H", RUN_TIME_SIZES)
+def test_run_time_radix_passes(ctx, W, H):
+    """Forward and inverse transforms by run-time radices against numpy in
+    FP64, and the same bits for rows of odd pitch at a 4-byte-aligned
+    address as for dense ones.  A convolution is two transforms of length
+    M < 4n and three products: about 2 (log2 M) / 2 + 3 roundings of 6e-8 on
+    the way, under 2e-6."""
+    import ctypes as C
+    print("run-time radices", W, H, flush=True)
+    rng = np.random.default_rng(W * 7 + H)
+    B = 2 if W * H < 3_000_000 else 1
+    x = rng.standard_normal((B, H, W)).astype(np.float32)
+    ref = np.fft.rfft2(x.astype(np.float64)).transpose(0, 2, 1)
+    spec = ctx.rfft2(ctx.upload(x))
+    assert _rel(spec.numpy(), ref) < 2e-6
+    half = ref.astype(np.complex64)
+    back = np.fft.irfft2(half.astype(np.complex128).transpose(0, 2, 1), s=(H, W)) * (W * H)
+    dense = ctx.irfft2(ctx.upload(half), W).numpy()
+    assert _rel(dense, back) < 2e-6
+    # odd pitch, one float into the buffer
+    pitch = W + 1
+    buf = np.zeros(B * H * pitch + 1, np.float32)
+    buf[1:].reshape(B, H, pitch)[:, :, :W] = x
+    d = ctx.upload(buf)
+    out = ctx.empty(spec.shape, np.complex64)
+    ctx._check(ctx.lib.mc_rfft2(ctx.ptr, d.vp(1), W, H, C.c_longlong(pitch), C.c_longlong(pitch * H), B,
+                                C.c_float(1.0), out.vp()), "mc_rfft2")
+    ctx.sync()
+    assert np.array_equal(out.numpy(), spec.numpy())
+    h = ctx.upload(half)
+    d = ctx.upload(np.full_like(buf, -7.0))
+    ctx._check(ctx.lib.mc_irfft2(ctx.ptr, h.vp(), W, H, B, d.vp(1), C.c_longlong(pitch), C.c_longlong(pitch * H), 0),
+               "mc_irfft2")
+    ctx.sync()
+    got = d.numpy()
+    assert got[0] == -7.0 and np.all(got[1:].reshape(B, H, pitch)[:, :, W:] == -7.0)
+    assert np.array_equal(got[1:].reshape(B, H, pitch)[:, :, :W], dense)
+
+
+@pytest.mark.parametrize("W,H,ft_bin", [(1000, 600, 2.0), (740, 820, 1.5), (3838, 3710, 2.0)])
+def test_run_time_radix_crop(ctx, W, H, ft_bin):
+    """The Fourier crop in the inverse column pass (output sums at the -FtBin
+    size) by run-time radices against numpy in FP64."""
+    rng = np.random.default_rng(W)
+    x = rng.uniform(0.5, 1.5, (2, H, W))
+    spec = (np.fft.rfft2(x) / (W * H)).astype(np.complex64)
+    ow, oh = int(W / ft_bin) // 2 * 2, int(H / ft_bin) // 2 * 2
+    out = ctx.finalize_sums(ctx.upload(np.ascontiguousarray(spec.transpose(0, 2, 1))), W, ft_bin).numpy()
+    rows = np.arange(oh)
+    rows = np.where(rows > oh // 2, rows - oh + H, rows)
+    ref = np.fft.irfft2(spec.astype(np.complex128)[:, rows, : ow // 2 + 1], s=(oh, ow)) * (ow * oh)
+    assert out.shape == ref.shape
+    assert _rel(out, np.maximum(ref, 0)) < 2e-6
