@@ -1205,33 +1205,30 @@ __global__ __launch_bounds__(256) void k_patch_stats(double* s, const double* ce
 // frames inside.  Per pixel the reference forms w_p = exp(-100 r_p) for every
 // patch with r_p <= 0.6 (r in units of the frame size), skips bad patches,
 // sums w, w*sx, w*sy in patch order in FP32, divides, and gathers the pixel at
-// (int)(x - sx), (int)(y - sy) with 811*|.| mod N reflection.  Here the
-// weights of a 64x4-pixel tile are formed once for all frames.  A patch whose
-// weight is below 1e-14 of the largest weight among a frame's good patches
-// (r > r_min + 0.3224) for every pixel of the tile is left out: adding it
-// cannot change any of the FP32 sums (it is far below half an ulp), so the
-// kept patches, taken in the reference's order, give the same sums.  r_min
-// is taken over the patches that are good in every frame (bad_any clear), an
-// upper bound on every frame's nearest good patch; with none, every patch
-// within r <= 0.6 is kept.  The frame table holds
-// {ok*sx, ok*sy, ok} per kept patch (ok = 0 for a bad patch), so
-// fw = fma(w, ok, fw) and fsx = fma(w, ok*sx, fsx) reproduce the reference's
-// skip exactly; up to 16 kept patches the weights live in registers.
-#define MC_WARP_MAXP 64
-#ifndef MC_WARP_TX
-#define MC_WARP_TX 64
-#endif
-#ifndef MC_WARP_TY
-#define MC_WARP_TY 4
-#endif
-#define MC_WARP_NT (MC_WARP_TX * MC_WARP_TY)
-#ifndef MC_WARP_FCH
-#define MC_WARP_FCH 16
-#endif
-#define MC_WARP_KREG 16
+// (int)(x - sx), (int)(y - sy) with 811*|.| mod N reflection.
+//
+// Here a pixel's weights are formed once for all frames and stay in
+// registers.  A patch whose weight is below e^-25 = 1.4e-11 of the largest
+// weight among a frame's good patches (r > r_min + 0.25) for every pixel of
+// the tile is left out: half an ulp of the FP32 sums is 4000 times that.  The
+// kept patches, taken in the reference's order, give the same sums.  r_min is
+// bounded over the patches that are good in every frame (bad_any clear); with
+// none, every patch within r <= 0.6 is kept.
+//
+// What bounds it: one gather and one store per pixel and frame (HBM), and
+// about 45 vector instructions.  The frames' shifts of the kept patches (zero
+// for a bad patch, which leaves the sums as the reference's skip does) lie in
+// LDS, two patches per 16-byte broadcast.  (As scalar loads, one per patch
+// and frame, they took 3.03 ms at 5760 x 4092, 24 frames, 25 patches: the
+// scalar cache's rate.)  The quotients take one exact reciprocal per pixel and
+// a correction step per frame, which rounds as the division does; tiles whose
+// sources all lie inside the frame skip the edge checks.  That case: 2.37 ->
+// 1.40 ms (3.2 TB/s), vector units 78% busy.
 #ifndef MC_WARP_U
 #define MC_WARP_U 8
 #endif
+#define MC_WARP_NT 256   // four waves, each 64 pixels of one row
+#define MC_WARP_KREG 32  // kept patches with weights in registers
 
 struct WarpArgs {
     const float* R;
@@ -1239,268 +1236,334 @@ struct WarpArgs {
     long long pitch, fstride;
     int W, H, N, P;
     const float* cen;
-    const float* sh;
-    const unsigned char* bad;
+    const float* sh;             // N x P x 2, zero where bad
+    const unsigned char* bad;    // N x P
     unsigned long long bad_any;  // bit p: patch p is bad in some frame
+    float smax;                  // largest |shift| in sh; below 0: not finite or absurd
 };
 
-// Source offset (within a frame) of output pixel (x, y) for the weighted
-// shift sums of one frame.
-__device__ __forceinline__ int warp_src(int W, int H, int pitch, int x, int y, float fw, float fsx,
-                                        float fsy) {
-    if (fw > 0) {
-        fsx = fsx / fw;
-        fsy = fsy / fw;
-    }
-    // keep the gather index finite for non-finite or absurd shifts
-    if (!(fabsf(fsx) < 1e6f)) fsx = 0.f;
-    if (!(fabsf(fsy) < 1e6f)) fsy = 0.f;
-    int xs = (int)((float)x - fsx);
-    int ys = (int)((float)y - fsy);
-    if (xs < 0 || ys < 0 || xs >= W || ys >= H) {
-        xs = xs < 0 ? -xs : xs;
-        ys = ys < 0 ? -ys : ys;
-        xs = (int)((811LL * xs) % W);
-        ys = (int)((811LL * ys) % H);
-    }
-    return ys * pitch + xs;
+// a / b with r = 1 / b correctly rounded: the remainder of the approximate
+// quotient is exact, and the corrected one rounds as a / b does.
+__device__ __forceinline__ float div_by(float a, float b, float r) {
+    const float q = a * r;
+    return fmaf(fmaf(-b, q, a), r, q);
 }
 
-// Fill the table of frames f0..f0+nf-1 for the K (>= nk) kept patches;
-// fbad[fi] (cleared by the caller) becomes 1 when a kept patch is bad in
-// frame f0 + fi.
-__device__ __forceinline__ void warp_table(const WarpArgs& a, const int* klist, int nk, int K,
-                                           int f0, int nf, float4* tab, int* fbad) {
-    for (int e = threadIdx.x; e < nf * K; e += MC_WARP_NT) {
-        const int fi = e / K, q = e - fi * K;
-        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (q < nk) {
-            const int p = klist[q];
-            const long long o = (long long)(f0 + fi) * a.P + p;
-            if (!a.bad[o]) {
-                t.x = a.sh[2 * o];
-                t.y = a.sh[2 * o + 1];
-                t.z = 1.f;
-            } else {
-                fbad[fi] = 1;
+// Reflection of a source position outside the frame.
+__device__ __forceinline__ int warp_reflect(int W, int H, int pitch, int xs, int ys) {
+    xs = xs < 0 ? -xs : xs;
+    ys = ys < 0 ? -ys : ys;
+    return (int)((811LL * ys) % H) * pitch + (int)((811LL * xs) % W);
+}
+
+// Bits of the patches kept for the tile of `nx` x `ny` pixels at (x0, y0);
+// lane p looks at patch p.
+__device__ __forceinline__ unsigned long long warp_select(const WarpArgs& a, int x0, int y0, int nx, int ny) {
+    const int p = threadIdx.x & 63;
+    const bool live = p < a.P;
+    const float cx = live ? a.cen[2 * p] : 0.f, cy = live ? a.cen[2 * p + 1] : 0.f;
+    const float rw = 1.0f / (float)a.W, rh = 1.0f / (float)a.H;
+    const float xl = ((float)x0 - cx) * rw, xh = ((float)(x0 + nx - 1) - cx) * rw;
+    const float yl = ((float)y0 - cy) * rh, yh = ((float)(y0 + ny - 1) - cy) * rh;
+    // distance to the nearest and to the farthest point of the tile
+    const float nxd = fmaxf(fmaxf(xl, -xh), 0.f), nyd = fmaxf(fmaxf(yl, -yh), 0.f);
+    const float fxd = fmaxf(fabsf(xl), fabsf(xh)), fyd = fmaxf(fabsf(yl), fabsf(yh));
+    const float dn = sqrtf(nxd * nxd + nyd * nyd), df = sqrtf(fxd * fxd + fyd * fyd);
+    float rmin = (live && !((a.bad_any >> p) & 1ull)) ? df : 1e30f;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) rmin = fminf(rmin, __shfl_xor(rmin, o));
+    // shifts that are not finite count from every patch in reach
+    return __ballot(live && dn <= (a.smax < 0 ? 0.6001f : fminf(rmin + 0.25f, 0.6001f)));
+}
+
+// An upper bound of the patches any tile keeps: the same rule on 24 x 24
+// boxes that cover the frame (a tile inside a box keeps no patch that the box
+// does not; boxes overlap by a tile).
+int mc_warp_keep_max(const float* cen, unsigned long long bad_any, int W, int H, int P) {
+    const int bw = W / 24 + 64, bh = H / 24 + 4;
+    int most = 0;
+    for (int y0 = 0; y0 < H; y0 += bh - 3)
+        for (int x0 = 0; x0 < W; x0 += bw - 63) {
+            const float x1 = std::min(x0 + bw, W) - 1, y1 = std::min(y0 + bh, H) - 1;
+            float dn[MC_WARP_MAXP], rmin = 1e30f;
+            for (int p = 0; p < P; p++) {
+                const float xl = (x0 - cen[2 * p]) / W, xh = (x1 - cen[2 * p]) / W;
+                const float yl = (y0 - cen[2 * p + 1]) / H, yh = (y1 - cen[2 * p + 1]) / H;
+                dn[p] = std::hypot(std::max(std::max(xl, -xh), 0.f), std::max(std::max(yl, -yh), 0.f));
+                if (!((bad_any >> p) & 1ull))
+                    rmin = std::min(rmin, std::hypot(std::max(std::fabs(xl), std::fabs(xh)),
+                                                     std::max(std::fabs(yl), std::fabs(yh))));
             }
+            int n = 0;
+            // (a margin for the rounding of the device's distances)
+            for (int p = 0; p < P; p++) n += !(dn[p] > std::min(rmin + 0.25f, 0.6001f) + 1e-3f);
+            most = std::max(most, n);
         }
-        tab[e] = t;
-    }
+    return most;
 }
 
-// A frame without bad kept patches has fw = sum_q w_q, the same FMA chain
-// (fma(w, 1, fw) is w + fw) for every such frame: it is formed once.
-template <int K>
-__device__ __forceinline__ void warp_tile_reg(const WarpArgs& a, const int* klist, int nk,
-                                              float4* tab, int* fbad, int x, int y, bool live) {
-    float w[K];
-#pragma unroll
-    for (int q = 0; q < K; q++) {
-        w[q] = 0.f;
-        if (live && q < nk) {
-            const int p = klist[q];
-            const float ax = ((float)x - a.cen[2 * p]) / (float)a.W;
-            const float ay = ((float)y - a.cen[2 * p + 1]) / (float)a.H;
-            const float r = sqrtf(ax * ax + ay * ay);
-            w[q] = (r > 0.6f) ? 0.f : expf(-100.0f * r);
+__device__ __forceinline__ float warp_weight(const WarpArgs& a, int p, int x, int y, float rw, float rh) {
+    const float ax = div_by((float)x - a.cen[2 * p], (float)a.W, rw);
+    const float ay = div_by((float)y - a.cen[2 * p + 1], (float)a.H, rh);
+    const float r = sqrtf(ax * ax + ay * ay);
+    return (r > 0.6f) ? 0.f : expf(-100.0f * r);
+}
+
+// Frames per LDS table: row fi holds the kept patches' shifts in a frame (K
+// pairs, zero past the kept ones), bad[fi] the bits of kept patches bad in it.
+#define MC_WARP_FCH 32
+struct WarpTable {
+    float2* sh;
+    unsigned long long* bad;
+    unsigned char* klist;  // patch numbers of the kept patches
+    int K;
+};
+
+// Fill the rows of frames idx(f0) .. idx(f0 + nf - 1).  All threads call it.
+template <class Idx>
+__device__ __forceinline__ void warp_fill(const WarpArgs& a, const WarpTable& t, unsigned long long mask, int f0,
+                                          int nf, Idx idx) {
+    const int nk = __popcll(mask);
+    __syncthreads();
+    if (threadIdx.x < MC_WARP_FCH) t.bad[threadIdx.x] = 0;
+    if (threadIdx.x < 64 && ((mask >> threadIdx.x) & 1ull))
+        t.klist[__popcll(mask & ((1ull << threadIdx.x) - 1))] = (unsigned char)threadIdx.x;
+    __syncthreads();
+    for (int e = threadIdx.x; e < nf * t.K; e += MC_WARP_NT) {
+        const int fi = e / t.K, q = e - fi * t.K;
+        float2 s = make_float2(0.f, 0.f);
+        if (q < nk) {
+            const int p = t.klist[q];
+            const long long o = (long long)idx(f0 + fi) * a.P + p;
+            s = reinterpret_cast<const float2*>(a.sh)[o];
+            if (a.bad[o]) atomicOr(&t.bad[fi], 1ull << q);
         }
+        t.sh[e] = s;
     }
-    float fw_all = 0.f;
+    __syncthreads();
+}
+
+// How a tile finds its source pixels: ANY checks the shifts and the frame's
+// edges; SAFE shifts are finite and below 1e5; INNER also keeps every source
+// of the tile inside the frame.
+enum { WARP_ANY, WARP_SAFE, WARP_INNER };
+
+// Source offset (within a frame) of output pixel (x, y) from the weight sum
+// (fw > 0; with inv = 1 / fw) and the weighted shift sums of one frame.
+template <int HOW>
+__device__ __forceinline__ int warp_src(const WarpArgs& a, int x, int y, float fw, float inv, float fsx, float fsy) {
+    fsx = div_by(fsx, fw, inv);
+    fsy = div_by(fsy, fw, inv);
+    if constexpr (HOW == WARP_ANY) {
+        // keep the gather index finite for non-finite or absurd shifts
+        if (!(fabsf(fsx) < 1e6f)) fsx = 0.f;
+        if (!(fabsf(fsy) < 1e6f)) fsy = 0.f;
+    }
+    const int xs = (int)((float)x - fsx);
+    const int ys = (int)((float)y - fsy);
+    if constexpr (HOW != WARP_INNER)
+        if ((unsigned)xs >= (unsigned)a.W || (unsigned)ys >= (unsigned)a.H)
+            return warp_reflect(a.W, a.H, (int)a.pitch, xs, ys);
+    return ys * (int)a.pitch + xs;
+}
+
+// A pixel's weights over K kept patches (K even), and its source offset in the
+// frame of a table row.
+template <int K>
+struct WarpPixel {
+    float w[K];
+    float fw, inv;  // weight sum of frames without a bad kept patch
+    int x, y;
+
+    __device__ __forceinline__ void init(const WarpArgs& a, unsigned long long mask, int px, int py, float*) {
+        const float rw = 1.0f / (float)a.W, rh = 1.0f / (float)a.H;
+        x = px;
+        y = py;
+        unsigned long long m = mask;
+        int p = 0;
 #pragma unroll
-    for (int q = 0; q < K; q++) fw_all = fmaf(w[q], q < nk ? 1.f : 0.f, fw_all);
-    for (int f0 = 0; f0 < a.N; f0 += MC_WARP_FCH) {
-        const int nf = min(MC_WARP_FCH, a.N - f0);
-        __syncthreads();
-        if (threadIdx.x < MC_WARP_FCH) fbad[threadIdx.x] = 0;
-        __syncthreads();
-        warp_table(a, klist, nk, K, f0, nf, tab, fbad);
-        __syncthreads();
-        if (!live) continue;
-        // gathers of MC_WARP_U frames are issued before their stores so that
-        // each wave keeps several loads in flight, and the next group's
-        // source offsets are formed while they are; offsets within a frame
-        // are 32-bit (the host checks pitch * H < 2^31)
-        const int pitch = (int)a.pitch;
-        const int oo = y * pitch + x;
-        int so[MC_WARP_U];
-        auto offsets = [&](int fb) {
+        for (int q = 0; q < K; q++) {
+            const bool on = m != 0;
+            if (on) p = __ffsll(m) - 1;
+            m &= m - 1;  // (zero stays zero)
+            w[q] = on ? warp_weight(a, p, x, y, rw, rh) : 0.f;
+        }
+        fw = 0.f;
+#pragma unroll
+        for (int q = 0; q < K; q++) fw += w[q];
+        recip(fw, fw, inv);
+    }
+    // a weight sum of zero leaves the shift sums as they are
+    static __device__ __forceinline__ void recip(float s, float& d, float& r) {
+        d = s > 0 ? s : 1.f;
+        r = 1.0f / d;
+    }
+    template <int HOW, bool BAD>
+    __device__ __forceinline__ int source(const WarpArgs& a, const WarpTable& t, int fi) const {
+        const float4* s = reinterpret_cast<const float4*>(t.sh) + fi * (K / 2);
+        float fsx = 0.f, fsy = 0.f;
+#pragma unroll
+        for (int q = 0; q < K / 2; q++) {
+            const float4 v = s[q];
+            fsx = fmaf(v.x, w[2 * q], fsx);
+            fsy = fmaf(v.y, w[2 * q], fsy);
+            fsx = fmaf(v.z, w[2 * q + 1], fsx);
+            fsy = fmaf(v.w, w[2 * q + 1], fsy);
+        }
+        float d = fw, r = inv;
+        if constexpr (BAD) {
+            const unsigned long long b = t.bad[fi];
+            float g = 0.f;
+#pragma unroll
+            for (int q = 0; q < K; q++) g += (b >> q) & 1ull ? 0.f : w[q];
+            recip(g, d, r);
+        }
+        return warp_src<HOW>(a, x, y, d, r, fsx, fsy);
+    }
+};
+
+// More kept patches than registers hold: weights in LDS, [q][thread].
+struct WarpPixelLds {
+    float* wk;
+    int nk, x, y;
+
+    __device__ __forceinline__ void init(const WarpArgs& a, unsigned long long mask, int px, int py, float* lds) {
+        wk = lds + threadIdx.x;
+        const float rw = 1.0f / (float)a.W, rh = 1.0f / (float)a.H;
+        x = px;
+        y = py;
+        nk = 0;
+        for (unsigned long long m = mask; m; m &= m - 1)
+            wk[MC_WARP_NT * nk++] = warp_weight(a, __ffsll(m) - 1, x, y, rw, rh);
+    }
+    template <int HOW, bool BAD>
+    __device__ __forceinline__ int source(const WarpArgs& a, const WarpTable& t, int fi) const {
+        const float2* s = t.sh + fi * t.K;
+        const unsigned long long b = t.bad[fi];
+        float fsx = 0.f, fsy = 0.f, g = 0.f, d, r;
+        for (int q = 0; q < nk; q++) {
+            const float w = wk[MC_WARP_NT * q];
+            // (a patch out of reach may have a shift that is not finite)
+            fsx = w > 0 ? fmaf(s[q].x, w, fsx) : fsx;
+            fsy = w > 0 ? fmaf(s[q].y, w, fsy) : fsy;
+            g += (b >> q) & 1ull ? 0.f : w;
+        }
+        WarpPixel<2>::recip(g, d, r);
+        return warp_src<HOW>(a, x, y, d, r, fsx, fsy);
+    }
+};
+
+// Gather the pixel from `cnt` frames, frame i being idx(i), and hand groups of
+// up to MC_WARP_U values to use(first i, count, values).  The next group's
+// gathers go out before this group is used: loads and stores share one memory
+// counter in issue order, so a wave waits only for the loads it uses, while
+// the previous group's stores stay in flight.  (The last group of a table
+// repeats its last frame in place of missing ones.)
+// Offsets within a frame are 32-bit byte offsets from a scalar base, except in
+// frames of 2^30 pixels and more (WIDE).
+template <int HOW, bool WIDE, class Px, class Idx, class Use>
+__device__ __forceinline__ void warp_frames(const WarpArgs& a, const Px& px, const WarpTable& t,
+                                            unsigned long long mask, int cnt, Idx idx, Use use) {
+    for (int f0 = 0; f0 < cnt; f0 += MC_WARP_FCH) {
+        const int nf = min(MC_WARP_FCH, cnt - f0);
+        warp_fill(a, t, mask, f0, nf, idx);
+        auto load = [&](int i0, float* d) {
+            int so[MC_WARP_U];
+            // frames with a bad kept patch sum their own weights; chosen per
+            // group, so that the groups without one are straight-line code
+            unsigned long long b = 0;
+#pragma unroll
+            for (int u = 0; u < MC_WARP_U; u++) b |= t.bad[min(i0 + u, nf - 1)];
+            if (__builtin_amdgcn_readfirstlane((int)(b | b >> 32))) {
+#pragma unroll
+                for (int u = 0; u < MC_WARP_U; u++) so[u] = px.template source<HOW, true>(a, t, min(i0 + u, nf - 1));
+            } else {
+#pragma unroll
+                for (int u = 0; u < MC_WARP_U; u++) so[u] = px.template source<HOW, false>(a, t, min(i0 + u, nf - 1));
+            }
 #pragma unroll
             for (int u = 0; u < MC_WARP_U; u++) {
-                const int fi = min(fb + u, nf - 1);
-                const float4* t = tab + fi * K;
-                float fw = fw_all, fsx = 0.f, fsy = 0.f;
-                if (fbad[fi]) {
-                    fw = 0.f;
-#pragma unroll
-                    for (int q = 0; q < K; q++) fw = fmaf(w[q], t[q].z, fw);
-                }
-#pragma unroll
-                for (int q = 0; q < K; q++) {
-                    const float4 v = t[q];
-                    fsx = fmaf(v.x, w[q], fsx);
-                    fsy = fmaf(v.y, w[q], fsy);
-                }
-                so[u] = warp_src(a.W, a.H, pitch, x, y, fw, fsx, fsy);
+                const float* __restrict__ fr = a.R + (long long)idx(f0 + min(i0 + u, nf - 1)) * a.fstride;
+                if constexpr (WIDE) d[u] = fr[so[u]];
+                else d[u] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(fr) + ((unsigned)so[u] << 2));
             }
         };
-        // Whole groups load and store without per-frame conditions: a
-        // conditional store sits in a block of its own, and the compiler
-        // then waits for every outstanding memory operation (the previous
-        // stores included) before it.  The last nf % MC_WARP_U frames go one
-        // at a time.
-        const int nfull = nf - nf % MC_WARP_U;
-        // Software-pipelined: group g+1's gathers go out before group g's
-        // stores.  Loads and stores share one memory counter, counted in
-        // issue order, so a wave then waits only for the loads it is about
-        // to store, while the previous group's stores stay in flight.
-        if (nfull) {
-            offsets(0);
-            float v[MC_WARP_U];
+        float v[MC_WARP_U];
+        load(0, v);
+        for (int i0 = 0; i0 < nf; i0 += MC_WARP_U) {
+            float vn[MC_WARP_U];
+            if (i0 + MC_WARP_U < nf) load(i0 + MC_WARP_U, vn);
+            use(f0 + i0, min(MC_WARP_U, nf - i0), v);
 #pragma unroll
-            for (int u = 0; u < MC_WARP_U; u++) v[u] = (a.R + (long long)(f0 + u) * a.fstride)[so[u]];
-            for (int fb = 0; fb + MC_WARP_U < nfull; fb += MC_WARP_U) {
-                offsets(fb + MC_WARP_U);
-                float vn[MC_WARP_U];
+            for (int u = 0; u < MC_WARP_U; u++) v[u] = vn[u];
+        }
+    }
+}
+
+template <int HOW, bool WIDE, class Px>
+__device__ __forceinline__ void warp_store(const WarpArgs& a, const WarpTable& t, unsigned long long mask, int x,
+                                           int y, float* lds = nullptr) {
+    Px px;
+    px.init(a, mask, x, y, lds);
+    float* __restrict__ out = a.Rp + (long long)y * a.pitch + x;
+    warp_frames<HOW, WIDE>(a, px, t, mask, a.N, [](int i) { return i; }, [&](int i0, int n, const float* v) {
+        if (n == MC_WARP_U) {
+            // unconditional stores: a conditional one sits in a block of its
+            // own, where the compiler waits for every outstanding access
 #pragma unroll
-                for (int u = 0; u < MC_WARP_U; u++)
-                    vn[u] = (a.R + (long long)(f0 + fb + MC_WARP_U + u) * a.fstride)[so[u]];
-#pragma unroll
-                for (int u = 0; u < MC_WARP_U; u++) (a.Rp + (long long)(f0 + fb + u) * a.fstride)[oo] = v[u];
-#pragma unroll
-                for (int u = 0; u < MC_WARP_U; u++) v[u] = vn[u];
-            }
+            for (int u = 0; u < MC_WARP_U; u++) out[(long long)(i0 + u) * a.fstride] = v[u];
+        } else {
 #pragma unroll
             for (int u = 0; u < MC_WARP_U; u++)
-                (a.Rp + (long long)(f0 + nfull - MC_WARP_U + u) * a.fstride)[oo] = v[u];
+                if (u < n) out[(long long)(i0 + u) * a.fstride] = v[u];
         }
-        for (int fi = nfull; fi < nf; fi++) {
-            const float4* t = tab + fi * K;
-            float fw = fw_all, fsx = 0.f, fsy = 0.f;
-            if (fbad[fi]) {
-                fw = 0.f;
-#pragma unroll
-                for (int q = 0; q < K; q++) fw = fmaf(w[q], t[q].z, fw);
-            }
-#pragma unroll
-            for (int q = 0; q < K; q++) {
-                const float4 v = t[q];
-                fsx = fmaf(v.x, w[q], fsx);
-                fsy = fmaf(v.y, w[q], fsy);
-            }
-            const long long fo = (long long)(f0 + fi) * a.fstride;
-            a.Rp[fo + oo] = a.R[fo + warp_src(a.W, a.H, pitch, x, y, fw, fsx, fsy)];
-        }
-    }
+    });
 }
 
-// More than MC_WARP_KREG kept patches: weights in LDS, run-time loop.
-__device__ __forceinline__ void warp_tile_lds(const WarpArgs& a, const int* klist, int nk,
-                                           float4* tab, int* fbad, float* wk, int x, int y, bool live) {
-    for (int q = 0; q < nk; q++) {
-        float w = 0.f;
-        if (live) {
-            const int p = klist[q];
-            const float ax = ((float)x - a.cen[2 * p]) / (float)a.W;
-            const float ay = ((float)y - a.cen[2 * p + 1]) / (float)a.H;
-            const float r = sqrtf(ax * ax + ay * ay);
-            w = (r > 0.6f) ? 0.f : expf(-100.0f * r);
-        }
-        wk[q * MC_WARP_NT + threadIdx.x] = w;
-    }
-    for (int f0 = 0; f0 < a.N; f0 += MC_WARP_FCH) {
-        const int nf = min(MC_WARP_FCH, a.N - f0);
-        __syncthreads();
-        warp_table(a, klist, nk, nk, f0, nf, tab, fbad);
-        __syncthreads();
-        if (!live) continue;
-        for (int fi = 0; fi < nf; fi++) {
-            const float4* t = tab + fi * nk;
-            float fw = 0.f, fsx = 0.f, fsy = 0.f;
-            for (int q = 0; q < nk; q++) {
-                const float4 v = t[q];
-                const float wq = wk[q * MC_WARP_NT + threadIdx.x];
-                fw = fmaf(wq, v.z, fw);
-                fsx = fmaf(v.x, wq, fsx);
-                fsy = fmaf(v.y, wq, fsy);
-            }
-            const long long fo = (long long)(f0 + fi) * a.fstride;
-            a.Rp[fo + (long long)y * a.pitch + x] =
-                a.R[fo + warp_src(a.W, a.H, (int)a.pitch, x, y, fw, fsx, fsy)];
-        }
-    }
-}
+// Launches by the number of kept patches of a tile (uniform over a workgroup):
+// up to 16 and up to 32 with weights in registers, more (or shifts that need
+// every check) with weights in LDS.  One kernel for all would give every tile
+// the registers of the largest variant (172 against 120, two waves per SIMD
+// for four); a tile of another class leaves after the selection.
+__host__ __device__ constexpr int warp_class(int nk) { return nk <= 16 ? 0 : nk <= MC_WARP_KREG ? 1 : 2; }
 
-// Dynamic LDS: frame table MC_WARP_FCH x max(K) float4, then (only when the
-// patch count exceeds MC_WARP_KREG) weights [kept patch][thread].
-__global__ __launch_bounds__(MC_WARP_NT) void k_local_warp(WarpArgs a) {
-    extern __shared__ float4 tab[];
-    __shared__ unsigned int kmask[2];
-    __shared__ int klist[MC_WARP_MAXP];
-    __shared__ int nk_s;
-    __shared__ int fbad[MC_WARP_FCH];
-    const int x = blockIdx.x * MC_WARP_TX + (threadIdx.x % MC_WARP_TX);
-    const int y = blockIdx.y * MC_WARP_TY + (threadIdx.x / MC_WARP_TX);
-    const bool live = x < a.W && y < a.H;
-    if (threadIdx.x == 0) kmask[0] = kmask[1] = 0u;
-    __syncthreads();
-    // Selection only has to be a superset of the patches that can matter, so
-    // it uses squared distances with reciprocal scales and a small margin;
-    // the weights themselves are computed exactly as the reference does.
-    const float rw = 1.0f / (float)a.W, rh = 1.0f / (float)a.H;
-    float r2min = 1e30f;
-    for (int p = 0; p < a.P && live; p++) {
-        if ((a.bad_any >> p) & 1ull) continue;
-        const float ax = ((float)x - a.cen[2 * p]) * rw;
-        const float ay = ((float)y - a.cen[2 * p + 1]) * rh;
-        r2min = fminf(r2min, ax * ax + ay * ay);
+// Tiles of 64 x 4 pixels, a wave per row.  Threads past the frame's edge repeat
+// its last pixel and store the same value to the same place.
+template <int CLASS, bool WIDE>
+__global__ __launch_bounds__(MC_WARP_NT, CLASS == 0 ? 4 : 2) void k_local_warp(WarpArgs a) {
+    const int x0 = blockIdx.x * 64, y0 = blockIdx.y * 4;
+    const int x = min((int)(x0 + (threadIdx.x & 63)), a.W - 1), y = min((int)(y0 + (threadIdx.x >> 6)), a.H - 1);
+    const unsigned long long mask = warp_select(a, x0, y0, min(64, a.W - x0), min(4, a.H - y0));
+    const int nk = __popcll(mask);
+    if (warp_class(nk) != CLASS && !(CLASS == 2 && a.smax < 0)) return;
+    constexpr int KMAX = CLASS == 0 ? 16 : CLASS == 1 ? MC_WARP_KREG : MC_WARP_MAXP;
+    __shared__ float4 tab[MC_WARP_FCH * KMAX / 2];
+    __shared__ unsigned long long bad[MC_WARP_FCH];
+    __shared__ unsigned char klist[MC_WARP_MAXP];
+    WarpTable t{reinterpret_cast<float2*>(tab), bad, klist, 0};
+    const float m = a.smax + 1.f;
+    const bool inner = x0 >= m && y0 >= m && x0 + 63 < a.W - m && y0 + 3 < a.H - m;
+#define MC_WK(KK)                                                                                    \
+    if (nk <= KK) {                                                                                  \
+        t.K = KK;                                                                                    \
+        if (inner) warp_store<WARP_INNER, WIDE, WarpPixel<KK>>(a, t, mask, x, y);                    \
+        else warp_store<WARP_SAFE, WIDE, WarpPixel<KK>>(a, t, mask, x, y);                           \
+        return;                                                                                      \
     }
-    const float rlim = fminf(sqrtf(r2min) + 0.3225f, 0.6001f);
-    const float r2lim = rlim * rlim;
-    unsigned int lo = 0u, hi = 0u;
-    for (int p = 0; p < a.P && live; p++) {
-        const float ax = ((float)x - a.cen[2 * p]) * rw;
-        const float ay = ((float)y - a.cen[2 * p + 1]) * rh;
-        if (ax * ax + ay * ay <= r2lim) {
-            if (p < 32) lo |= 1u << p;
-            else hi |= 1u << (p - 32);
-        }
+    if constexpr (CLASS == 0) {
+        MC_WK(4) MC_WK(6) MC_WK(8) MC_WK(10) MC_WK(12) MC_WK(16)
+    } else if constexpr (CLASS == 1) {
+        MC_WK(24) MC_WK(32)
+    } else {
+        extern __shared__ float warp_lds[];
+        t.K = MC_WARP_MAXP;
+        warp_store<WARP_ANY, WIDE, WarpPixelLds>(a, t, mask, x, y, warp_lds);
     }
-    if (lo) atomicOr(&kmask[0], lo);
-    if (hi) atomicOr(&kmask[1], hi);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int n = 0;
-        for (int p = 0; p < a.P; p++) {
-            const unsigned int wd = kmask[p >> 5];
-            if ((wd >> (p & 31)) & 1u) klist[n++] = p;
-        }
-        nk_s = n;
-    }
-    __syncthreads();
-    const int nk = nk_s;
-    switch (nk) {
-#define MC_WK(K) \
-    case K: warp_tile_reg<K>(a, klist, nk, tab, fbad, x, y, live); return;
-        MC_WK(1) MC_WK(2) MC_WK(3) MC_WK(4) MC_WK(5) MC_WK(6) MC_WK(7) MC_WK(8)
-        MC_WK(9) MC_WK(10) MC_WK(11) MC_WK(12) MC_WK(13) MC_WK(14) MC_WK(15) MC_WK(16)
 #undef MC_WK
-        default: break;
-    }
-    if (nk == 0) {
-        warp_tile_reg<1>(a, klist, 0, tab, fbad, x, y, live);
-        return;
-    }
-        warp_tile_lds(a, klist, nk, tab, fbad, reinterpret_cast<float*>(tab + MC_WARP_FCH * a.P), x, y,
-                      live);
 }
 
-static size_t warp_lds_bytes(int P) {
-    const int kt = P > MC_WARP_KREG ? P : MC_WARP_KREG;
-    size_t b = (size_t)MC_WARP_FCH * kt * sizeof(float4);
-    if (P > MC_WARP_KREG) b += (size_t)P * MC_WARP_NT * sizeof(float);
-    return b;
-}
+// Weights in LDS of the workgroups that keep more patches than registers hold.
+static size_t warp_lds_bytes(int P) { return (size_t)P * MC_WARP_NT * sizeof(float); }
 
 // ---------------------------------------------------------------------------
 // CCorrectFullShift::mGenSums (Correct/CCorrectFullShift.cpp:271-300) over
@@ -1686,8 +1749,10 @@ int mc_align_init_constants() {
     attr_ok &= hipSuccess == hipFuncSetAttribute((const void*)k_row_dft, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     attr_ok &= hipSuccess == hipFuncSetAttribute((const void*)k_feature_map, hipFuncAttributeMaxDynamicSharedMemorySize,
                         2 * 128 * 128 * (int)sizeof(float));
-    attr_ok &= hipSuccess == hipFuncSetAttribute((const void*)k_local_warp, hipFuncAttributeMaxDynamicSharedMemorySize,
-                        (int)warp_lds_bytes(MC_WARP_MAXP));
+    attr_ok &= hipSuccess == hipFuncSetAttribute((const void*)k_local_warp<2, false>,
+                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)warp_lds_bytes(MC_WARP_MAXP));
+    attr_ok &= hipSuccess == hipFuncSetAttribute((const void*)k_local_warp<2, true>,
+                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)warp_lds_bytes(MC_WARP_MAXP));
     return attr_ok ? 0 : -1;
 }
 
@@ -1899,12 +1964,22 @@ hipError_t mc_launch_patch_stats(double* shifts, const double* centers, int N, i
 
 hipError_t mc_launch_local_warp(const float* R, float* Rp, long long pitch, long long fstride,
                                 int W, int H, int N, int P, const float* cen, const float* sh,
-                                const unsigned char* bad, unsigned long long bad_any, hipStream_t s) {
-    if (P < 1 || P > MC_WARP_MAXP) return hipErrorInvalidValue;
+                                const unsigned char* bad, unsigned long long bad_any, int keep_max,
+                                float smax, hipStream_t s) {
+    if (P < 1 || P > MC_WARP_MAXP || keep_max < 0) return hipErrorInvalidValue;
     if (pitch * H >= (1LL << 31) || pitch < W) return hipErrorInvalidValue;
-    WarpArgs a{R, Rp, pitch, fstride, W, H, N, P, cen, sh, bad, bad_any};
-    dim3 grid(mc_div_up(W, MC_WARP_TX), mc_div_up(H, MC_WARP_TY));
-    hipLaunchKernelGGL(k_local_warp, grid, dim3(MC_WARP_NT), warp_lds_bytes(P), s, a);
+    WarpArgs a{R, Rp, pitch, fstride, W, H, N, P, cen, sh, bad, bad_any, smax};
+    const dim3 grid(mc_div_up(W, 64), mc_div_up(H, 4)), blk(MC_WARP_NT);
+    const size_t lds = warp_lds_bytes(P);
+    const int top = warp_class(keep_max);
+    const bool wide = pitch * H >= (1LL << 30);
+#define X(CL)                                                                                        \
+    if (smax < 0 ? CL == 2 : top >= CL) {                                                            \
+        if (wide) hipLaunchKernelGGL((k_local_warp<CL, true>), grid, blk, CL == 2 ? lds : 0, s, a);  \
+        else hipLaunchKernelGGL((k_local_warp<CL, false>), grid, blk, CL == 2 ? lds : 0, s, a);      \
+    }
+    X(0) X(1) X(2)
+#undef X
     return hipGetLastError();
 }
 

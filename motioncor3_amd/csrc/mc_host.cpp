@@ -319,6 +319,23 @@ unsigned long long bad_any_of(const unsigned char* bad, int N, int P) {
     return m;
 }
 
+// The local warp's view of an N x P x 2 shift table: zero where a patch is
+// bad, and its largest magnitude (-1 when a shift is not finite or above 1e5).
+struct WarpShifts {
+    std::vector<float> s;
+    float most = 0.f;
+    WarpShifts(const float* shifts, const unsigned char* bad, int N, int P)
+        : s(shifts, shifts + 2 * (size_t)N * P) {
+        bool safe = true;
+        for (size_t e = 0; e < s.size(); e++) {
+            if (bad && bad[e / 2]) s[e] = 0.f;
+            if (!(std::fabs(s[e]) <= 1e5f)) safe = false;
+            most = std::max(most, std::fabs(s[e]));
+        }
+        if (!safe) most = -1.f;
+    }
+};
+
 // ---------------------------------------------------------------------------
 // geometry: CBufferPool.cpp:185-262, Align/CAlignBase.cpp:41-47
 struct Geo {
@@ -1774,16 +1791,18 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             std::vector<float> psf(ps.size()), pcf(pc.size());
             for (size_t i = 0; i < ps.size(); i++) psf[i] = (float)ps[i];
             for (size_t i = 0; i < pc.size(); i++) pcf[i] = (float)pc[i];
+            const WarpShifts wsh(psf.data(), bad.data(), N, P);
             MC_BUF(dpsf, float, "psf", psf.size());
             MC_BUF(dpcf, float, "pcf", pcf.size());
             MC_BUF(dbad2, unsigned char, "bad2", bad.size());
-            MC_TRY(hipMemcpyAsync(dpsf, psf.data(), sizeof(float) * psf.size(), hipMemcpyHostToDevice, s));
+            MC_TRY(hipMemcpyAsync(dpsf, wsh.s.data(), sizeof(float) * psf.size(), hipMemcpyHostToDevice, s));
             MC_TRY(hipMemcpyAsync(dpcf, pcf.data(), sizeof(float) * pcf.size(), hipMemcpyHostToDevice, s));
             MC_TRY(hipMemcpyAsync(dbad2, bad.data(), bad.size(), hipMemcpyHostToDevice, s));
             {
                 KTimer kt(c, "local_warp");
-                MC_TRY(mc_launch_local_warp(Rr, Rw, W, rfs, W, H, N, P, dpcf, dpsf, dbad2,
-                                            bad_any_of(bad.data(), N, P), s));
+                const unsigned long long any = bad_any_of(bad.data(), N, P);
+                MC_TRY(mc_launch_local_warp(Rr, Rw, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any,
+                                            mc_warp_keep_max(pcf.data(), any, W, H, P), wsh.most, s));
             }
             MC_TRY(fork());
             for (int f0 = 0; f0 < N; f0 += CH) {
@@ -2402,11 +2421,13 @@ int mc_local_warp(mc_ctx* c, const float* in, float* out, int W, int H, int N, i
     MC_BUF(ds, float, "api_ws", (size_t)2 * N * P);
     MC_BUF(db, unsigned char, "api_wb", (size_t)N * P);
     MC_TRY(hipMemcpyAsync(dc, centers, sizeof(float) * 2 * P, hipMemcpyHostToDevice, c->stream));
-    MC_TRY(hipMemcpyAsync(ds, shifts, sizeof(float) * 2 * N * P, hipMemcpyHostToDevice, c->stream));
+    const WarpShifts sh(shifts, bad, N, P);
+    MC_TRY(hipMemcpyAsync(ds, sh.s.data(), sizeof(float) * 2 * N * P, hipMemcpyHostToDevice, c->stream));
     if (bad) MC_TRY(hipMemcpyAsync(db, bad, (size_t)N * P, hipMemcpyHostToDevice, c->stream));
     else MC_TRY(hipMemsetAsync(db, 0, (size_t)N * P, c->stream));
-    MC_TRY(mc_launch_local_warp(in, out, W, (long long)W * H, W, H, N, P, dc, ds, db, bad_any_of(bad, N, P),
-                                c->stream));
+    const unsigned long long any = bad_any_of(bad, N, P);
+    MC_TRY(mc_launch_local_warp(in, out, W, (long long)W * H, W, H, N, P, dc, ds, db, any,
+                                mc_warp_keep_max(centers, any, W, H, P), sh.most, c->stream));
     return MC_OK;
 }
 
@@ -2437,12 +2458,14 @@ int mc_local_warp_noalloc(mc_ctx* c, const float* in, float* out, int W, int H, 
     float* ds = (float*)(c->scratch + os);
     unsigned char* db = c->scratch + ob;
     MC_TRY(hipMemcpyAsync(dc, centers, sizeof(float) * 2 * P, hipMemcpyHostToDevice, c->stream));
-    MC_TRY(hipMemcpyAsync(ds, shifts, sizeof(float) * 2 * (size_t)N * P, hipMemcpyHostToDevice, c->stream));
+    const WarpShifts sh(shifts, bad, N, P);
+    MC_TRY(hipMemcpyAsync(ds, sh.s.data(), sizeof(float) * 2 * (size_t)N * P, hipMemcpyHostToDevice, c->stream));
     // the previous call's flags are still there: write or clear all of them
     if (bad) MC_TRY(hipMemcpyAsync(db, bad, (size_t)N * P, hipMemcpyHostToDevice, c->stream));
     else MC_TRY(mc_launch_fill_u8(db, (long long)N * P, 0, c->stream));
-    MC_TRY(mc_launch_local_warp(in, out, W, (long long)W * H, W, H, N, P, dc, ds, db, bad_any_of(bad, N, P),
-                                c->stream));
+    const unsigned long long any = bad_any_of(bad, N, P);
+    MC_TRY(mc_launch_local_warp(in, out, W, (long long)W * H, W, H, N, P, dc, ds, db, any,
+                                mc_warp_keep_max(centers, any, W, H, P), sh.most, c->stream));
     return MC_OK;
 }
 

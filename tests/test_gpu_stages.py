@@ -252,3 +252,71 @@ def test_finalize_sums_match_oracle(ctx, W, H, ft_bin):
         ref = np.maximum(O.irfft2(O.fourier_resize(specs[k].astype(np.complex128), ow // 2 + 1, oh), ow), 0)
         assert np.linalg.norm(out[k] - ref) / np.linalg.norm(ref) < 1e-5, k
         assert out[k].min() >= 0
+
+
+def _warp_fp32(img, cen, sh, bad):
+    """mGCorrect3D (Correct/GCorrectPatchShift.cu:17-66) in FP32, all patches
+    in order; non-finite or absurd quotients count as no shift."""
+    f = np.float32
+    N, H, W = img.shape
+    x, y = np.arange(W, dtype=f)[None, :], np.arange(H, dtype=f)[:, None]
+    w = []
+    for c in cen.astype(f):
+        ax, ay = (x - c[0]) / f(W), (y - c[1]) / f(H)
+        r = np.sqrt(ax * ax + ay * ay, dtype=f)
+        w.append(np.where(r > f(0.6), f(0), np.exp(f(-100) * r, dtype=f)))
+    out, edge = np.empty_like(img), np.zeros(img.shape, bool)
+    with np.errstate(all="ignore"):
+        for i in range(N):
+            fw, sx, sy = (np.zeros((H, W), f) for _ in range(3))
+            for p in range(len(cen)):
+                if not bad[i, p]:
+                    on = w[p] > 0  # within r <= 0.6
+                    fw = fw + w[p]
+                    sx = np.where(on, sx + w[p] * f(sh[i, p, 0]), sx)
+                    sy = np.where(on, sy + w[p] * f(sh[i, p, 1]), sy)
+            sx, sy = (np.where(fw > 0, s / np.where(fw > 0, fw, f(1)), s) for s in (sx, sy))
+            sx, sy = (np.where(np.abs(s) < f(1e6), s, f(0)) for s in (sx, sy))
+            span = np.max(np.abs(sh[i]), initial=0.0, where=np.isfinite(sh[i])) + 1
+            for u, s in ((x, sx), (y, sy)):
+                d = u.astype(np.float64) - s
+                edge[i] |= (s != 0) & (np.abs(d - np.round(d)) < 1e-6 * np.abs(u) + 8e-6 * span)
+            xs, ys = np.trunc(x - sx).astype(np.int64), np.trunc(y - sy).astype(np.int64)
+            o = (xs < 0) | (ys < 0) | (xs >= W) | (ys >= H)
+            xs, ys = np.where(o, 811 * np.abs(xs) % W, xs), np.where(o, 811 * np.abs(ys) % H, ys)
+            out[i] = img[i][ys, xs]
+    return out, edge
+
+
+# frames of one partial tile, of several, with and without inner tiles; frame
+# counts below, at and above a gather group (8) and a shift table (32)
+@pytest.mark.parametrize("W,H,N", [(70, 9, 3), (333, 301, 8), (640, 402, 41)])
+@pytest.mark.parametrize("kind", ["grid3", "grid5", "cluster24", "cluster50", "far", "wild"])
+def test_local_warp_classes(ctx, W, H, N, kind):
+    """Every class of kept patches (up to 16, 32, more), tiles with no patch
+    in reach, bad patches, sources inside and outside the frame, and shifts
+    that need every check, against FP32 numpy.  One rounding of r (6e-8 of up
+    to 0.6) moves a weight exp(-100 r) by up to 4e-6, so the weighted shift
+    may move by 8e-6 of the frame's largest shift: a pixel may differ only
+    where its source is that near a pixel's edge."""
+    print("warp", W, H, N, kind, flush=True)
+    rng = np.random.default_rng(W + N)
+    if kind.startswith("grid"):
+        n = int(kind[4:])
+        cen = np.array([[(i % n + 0.5) * W / n, (i // n + 0.5) * H / n] for i in range(n * n)])
+    elif kind.startswith("cluster"):
+        cen = np.stack([rng.uniform(0.4, 0.6, int(kind[7:])) * W, rng.uniform(0.4, 0.6, int(kind[7:])) * H], 1)
+    else:
+        cen = np.array([[2.0 * W, 0.5 * H], [2.0 * W, 2.0 * H]]) if kind == "far" else \
+            np.array([[0.2 * W, 0.5 * H], [0.8 * W, 0.5 * H], [0.5 * W, 0.9 * H]])
+    P = len(cen)
+    sh = rng.normal(0, 2.5, (N, P, 2)).astype(np.float32)
+    bad = (rng.random((N, P)) < 0.1).astype(np.uint8)
+    if kind == "wild":
+        sh[0, 0], sh[1, 1], sh[2, 2] = np.nan, np.inf, 3e7
+        sh[1, 0] = -2.0 * W
+    img = rng.random((N, H, W)).astype(np.float32)
+    out = ctx.local_warp(ctx.upload(img), cen.astype(np.float32), sh, bad).numpy()
+    ref, edge = _warp_fp32(img, cen, sh, bad)
+    assert kind == "wild" or np.mean(edge) < 0.02
+    assert not np.any((out != ref) & ~edge)
