@@ -91,6 +91,20 @@ hipError_t mc_launch_local_warp(const float* R, float* Rp, long long pitch, long
                                 int W, int H, int N, int P, const float* cen, const float* sh,
                                 const unsigned char* bad, unsigned long long bad_any, int keep_max,
                                 float smax, hipStream_t s);
+// The warped frames added up instead of stored: plain (and even / odd) sums,
+// and MC_SUM_RANK-coefficient sums per class of frames (cls: first entry of
+// order, entries, nodes, first image, 0 / 1 for the even / odd sum or -1).
+#define MC_SUM_RANK 8
+bool mc_warp_sums_fit(long long pitch, int H, int keep_max, float smax);
+hipError_t mc_launch_warp_sums(const float* R, long long pitch, long long fstride, int W, int H, int N, int P,
+                               const float* cen, const float* sh, const unsigned char* bad,
+                               unsigned long long bad_any, int keep_max, float smax, const int* order,
+                               const float* lam, const int* cls, int ncls, float* img, float* plain, float* even,
+                               float* odd, int clamp, hipStream_t s);
+// Dose-weighted sum spectra from the node images' spectra G.
+hipError_t mc_launch_dw_nodes(const cfloat* G, long long gstride, int N, int cx, int H, double pix, double kvf,
+                              double dose, const int* cum, const int* node, const int* flags, int dws, int split,
+                              cfloat* sums, long long sstride, hipStream_t s);
 // keep_max of the above, from the patch centres on the host
 int mc_warp_keep_max(const float* cen, unsigned long long bad_any, int W, int H, int P);
 hipError_t mc_launch_dw_sums(const cfloat* F, long long fstride, int N, int cx, int H,

@@ -1562,6 +1562,95 @@ __global__ __launch_bounds__(MC_WARP_NT, CLASS == 0 ? 4 : 2) void k_local_warp(W
 #undef MC_WK
 }
 
+// ---------------------------------------------------------------------------
+// The corrected frames of patch mode go into few sums, so they are never
+// stored: the warp adds them up where it gathers them.  The plain sum needs no
+// transform at all.  The dose-weighted sums need sum_i q^c_i F_i with
+// q = exp(-0.5 dose / Dc(k)) different at every frequency; q^c as a function
+// of c is smooth, so over a class of frames q^c_i = sum_j lam_ij q^c_j holds
+// for a few node frames j to below FP32 rounding (SumPlan in mc_host.cpp),
+// and sum_i q^c_i F_i = sum_j q^c_j FFT(sum_i lam_ij frame_i): the transforms
+// run over one image per node, 16 instead of 50 at 1 e-/px and frame.
+// Bound by the gathers (4 B per pixel and frame) and the warp's vector work;
+// the accumulators add MC_SUM_RANK FMAs per pixel and frame.
+struct WarpSumArgs {
+    WarpArgs w;
+    const int* order;     // frames, class by class
+    const float* lam;     // MC_SUM_RANK coefficients per entry of order
+    const int* cls;       // per class: first entry, entries, nodes, first image, even/odd image or -1
+    int ncls;
+    float* img;           // node images, w.fstride apart
+    float* plain;         // plain sum
+    float* half[2];       // even / odd sums (or null)
+    int clamp;            // plain, half: max(0, .)
+};
+
+template <int HOW, class Px>
+__device__ __forceinline__ void warp_sum(const WarpSumArgs& s, const WarpTable& t, unsigned long long mask, int x,
+                                         int y) {
+    const WarpArgs& a = s.w;
+    Px px;
+    px.init(a, mask, x, y, nullptr);
+    const long long o = (long long)y * a.pitch + x;
+    float total = 0.f;
+    for (int c = 0; c < s.ncls; c++) {
+        const int* __restrict__ cl = s.cls + 5 * c;
+        const int first = cl[0], nodes = cl[2];
+        const int* __restrict__ order = s.order + first;
+        const float* __restrict__ lam = s.lam + first * MC_SUM_RANK;
+        float acc[MC_SUM_RANK], sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < MC_SUM_RANK; j++) acc[j] = 0.f;
+        warp_frames<HOW, false>(a, px, t, mask, cl[1], [&](int i) { return order[i]; },
+                                [&](int i0, int n, const float* v) {
+#pragma unroll
+            for (int u = 0; u < MC_WARP_U; u++) {
+                if (u >= n) break;
+                sum += v[u];
+                if (nodes)
+#pragma unroll
+                    for (int j = 0; j < MC_SUM_RANK; j++) acc[j] = fmaf(lam[(i0 + u) * MC_SUM_RANK + j], v[u], acc[j]);
+            }
+        });
+        float* __restrict__ im = s.img + cl[3] * a.fstride + o;
+#pragma unroll
+        for (int j = 0; j < MC_SUM_RANK; j++)
+            if (j < nodes) im[j * a.fstride] = acc[j];
+        if (cl[4] >= 0) s.half[cl[4]][o] = s.clamp ? fmaxf(sum, 0.f) : sum;
+        total += sum;
+    }
+    s.plain[o] = s.clamp ? fmaxf(total, 0.f) : total;
+}
+
+template <int CLASS>
+__global__ __launch_bounds__(MC_WARP_NT, CLASS == 0 ? 4 : 2) void k_warp_sums(WarpSumArgs s) {
+    const WarpArgs& a = s.w;
+    const int x0 = blockIdx.x * 64, y0 = blockIdx.y * 4;
+    const int x = min((int)(x0 + (threadIdx.x & 63)), a.W - 1), y = min((int)(y0 + (threadIdx.x >> 6)), a.H - 1);
+    const unsigned long long mask = warp_select(a, x0, y0, min(64, a.W - x0), min(4, a.H - y0));
+    const int nk = __popcll(mask);
+    if (warp_class(nk) != CLASS) return;
+    __shared__ float4 tab[MC_WARP_FCH * (CLASS == 0 ? 16 : MC_WARP_KREG) / 2];
+    __shared__ unsigned long long bad[MC_WARP_FCH];
+    __shared__ unsigned char klist[MC_WARP_MAXP];
+    WarpTable t{reinterpret_cast<float2*>(tab), bad, klist, 0};
+    const float m = a.smax + 1.f;
+    const bool inner = x0 >= m && y0 >= m && x0 + 63 < a.W - m && y0 + 3 < a.H - m;
+#define MC_WK(KK)                                                             \
+    if (nk <= KK) {                                                           \
+        t.K = KK;                                                             \
+        if (inner) warp_sum<WARP_INNER, WarpPixel<KK>>(s, t, mask, x, y);     \
+        else warp_sum<WARP_SAFE, WarpPixel<KK>>(s, t, mask, x, y);            \
+        return;                                                               \
+    }
+    if constexpr (CLASS == 0) {
+        MC_WK(4) MC_WK(6) MC_WK(8) MC_WK(10) MC_WK(12) MC_WK(16)
+    } else {
+        MC_WK(24) MC_WK(32)
+    }
+#undef MC_WK
+}
+
 // Weights in LDS of the workgroups that keep more patches than registers hold.
 static size_t warp_lds_bytes(int P) { return (size_t)P * MC_WARP_NT * sizeof(float); }
 
@@ -1652,6 +1741,63 @@ __global__ __launch_bounds__(256) void k_dw_sums(DwArgs a) {
         a.sums[(long long)(ns++) * a.sstride + q] = s1;
         if (a.dws) a.sums[(long long)(ns++) * a.sstride + q] = s2;
     }
+    if (a.split) {
+        a.sums[(long long)ns * a.sstride + q] = se;
+        a.sums[(long long)(ns + 1) * a.sstride + q] = so;
+    }
+}
+
+// The dose-weighted sums of k_dw_sums from node images (k_warp_sums): node
+// frame i's spectrum is image node[i], its weight the frame's own.  flags[i]:
+// bit 0 in -SumRange, bit 1 odd.
+struct DwNodeArgs {
+    const cfloat* G;
+    long long gstride;
+    int N, cx, H;
+    double pix, kvf, dose;
+    const int* cum;      // raw frames counted into frame i's dose
+    const int* node;     // image of frame i, or -1
+    const int* flags;
+    int dws, split;
+    cfloat* sums;        // _DW, then _DWS, even and odd as asked for
+    long long sstride;
+};
+
+__global__ __launch_bounds__(256) void k_dw_nodes(DwNodeArgs a) {
+    const int kx = blockIdx.y;
+    const int y = blockIdx.x * blockDim.x + threadIdx.x;
+    if (y >= a.H) return;
+    const long long q = (long long)kx * a.H + y;
+    double qd = 1.0, inv_ws = 1.0;
+    if (kx != 0 || y != 0) {
+        qd = crit_q(kx, y, a.cx, a.H, a.pix, a.kvf, a.dose);
+        double w = 1.0, s = 0.0;
+        int prev = 0;
+        for (int i = 0; i < a.N; i++) {
+            const int c = a.cum[i];
+            for (int k = prev; k < c; k++) w *= qd;
+            prev = c;
+            s += w * w;
+        }
+        inv_ws = 1.0 / sqrt(s);
+    }
+    cfloat s1 = cmk(0.f, 0.f), s2 = s1, so = s1, se = s1;
+    double w = 1.0;
+    int prev = 0;
+    for (int i = 0; i < a.N; i++) {
+        const int c = a.cum[i], nd = a.node[i], fl = a.flags[i];
+        for (int k = prev; k < c; k++) w *= qd;
+        prev = c;
+        if (nd < 0) continue;
+        const cfloat v = cscale(a.G[(long long)nd * a.gstride + q], (float)(w * inv_ws));
+        s1 = cadd(s1, v);
+        if (fl & 1) s2 = cadd(s2, v);
+        if (fl & 2) so = cadd(so, v);
+        else se = cadd(se, v);
+    }
+    int ns = 0;
+    a.sums[(long long)(ns++) * a.sstride + q] = s1;
+    if (a.dws) a.sums[(long long)(ns++) * a.sstride + q] = s2;
     if (a.split) {
         a.sums[(long long)ns * a.sstride + q] = se;
         a.sums[(long long)(ns + 1) * a.sstride + q] = so;
@@ -1980,6 +2126,34 @@ hipError_t mc_launch_local_warp(const float* R, float* Rp, long long pitch, long
     }
     X(0) X(1) X(2)
 #undef X
+    return hipGetLastError();
+}
+
+hipError_t mc_launch_warp_sums(const float* R, long long pitch, long long fstride, int W, int H, int N, int P,
+                               const float* cen, const float* sh, const unsigned char* bad,
+                               unsigned long long bad_any, int keep_max, float smax, const int* order,
+                               const float* lam, const int* cls, int ncls, float* img, float* plain, float* even,
+                               float* odd, int clamp, hipStream_t s) {
+    if (P < 1 || P > MC_WARP_MAXP || pitch * H >= (1LL << 30) || pitch < W || smax < 0 ||
+        warp_class(keep_max) > 1)
+        return hipErrorInvalidValue;
+    WarpSumArgs a{{R, nullptr, pitch, fstride, W, H, N, P, cen, sh, bad, bad_any, smax}, order, lam, cls, ncls, img,
+                  plain, {even, odd}, clamp};
+    const dim3 grid(mc_div_up(W, 64), mc_div_up(H, 4)), blk(MC_WARP_NT);
+    hipLaunchKernelGGL(k_warp_sums<0>, grid, blk, 0, s, a);
+    if (warp_class(keep_max) > 0) hipLaunchKernelGGL(k_warp_sums<1>, grid, blk, 0, s, a);
+    return hipGetLastError();
+}
+
+bool mc_warp_sums_fit(long long pitch, int H, int keep_max, float smax) {
+    return pitch * H < (1LL << 30) && smax >= 0 && warp_class(keep_max) <= 1;
+}
+
+hipError_t mc_launch_dw_nodes(const cfloat* G, long long gstride, int N, int cx, int H, double pix, double kvf,
+                              double dose, const int* cum, const int* node, const int* flags, int dws, int split,
+                              cfloat* sums, long long sstride, hipStream_t s) {
+    DwNodeArgs a{G, gstride, N, cx, H, pix, kvf, dose, cum, node, flags, dws, split, sums, sstride};
+    hipLaunchKernelGGL(k_dw_nodes, dim3(mc_div_up(H, 256), cx), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -17,6 +17,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -29,6 +30,7 @@
 #include "mc_ingest.h"
 #include "mc_output.h"
 #include "mc_prior.h"
+#include "mc_sums.h"
 #include "mc_tiff.h"
 
 // A learned shift prior on the context's device (mc_prior_create).
@@ -83,6 +85,9 @@ struct mc_ctx {
     hipEvent_t evt = nullptr;
     // learned prior for guided patch alignment (not owned)
     mc_prior* prior = nullptr;
+    // the last dose-weighted sum plan and what it was made for
+    std::unique_ptr<SumPlan> sum_plan;
+    SumPlanKey sum_key;
     // timing events of the stage clock (mc_result.seconds_stage), reused
     std::vector<hipEvent_t> stage_ev;
     // ingest: stream and completion event of asynchronous frame loads, and
@@ -1723,6 +1728,9 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
         float* gfm = gf ? gf + (long long)m * N : nullptr;
         float* ifm = iff ? iff + (long long)m * N : nullptr;
         MC_BUF(sums, cfloat, "sums", (size_t)nsum * fs);
+        // the output sums' spectra (null: that sum is done)
+        const cfloat* spec_sums[5];
+        for (int i = 0; i < nsum; i++) spec_sums[i] = sums + (long long)i * fs;
         MC_BUF(gsh, double, "gsh", 2 * N);
         MC_BUF(fA, cfloat, "fphA", (size_t)N * g.cx);
         MC_BUF(fB, cfloat, "fphB", (size_t)N * H);
@@ -1742,7 +1750,6 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             relative_to_ref(gshift.data(), N, p->fm_ref);
             // Correct/GCorrectPatchShift.cu:214-285: C2R, warp, normalised R2C
             MC_BUF(Rr, float, "Rr", (size_t)N * W * H);
-            MC_BUF(Rw, float, "Rw", (size_t)N * W * H);
             const long long rfs = (long long)W * H;
             if (early_inverse) {
                 // the chunks the early inverse left, on this stream, which
@@ -1792,41 +1799,138 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             for (size_t i = 0; i < ps.size(); i++) psf[i] = (float)ps[i];
             for (size_t i = 0; i < pc.size(); i++) pcf[i] = (float)pc[i];
             const WarpShifts wsh(psf.data(), bad.data(), N, P);
+            const unsigned long long any = bad_any_of(bad.data(), N, P);
+            const int keep = mc_warp_keep_max(pcf.data(), any, W, H, P);
             MC_BUF(dpsf, float, "psf", psf.size());
             MC_BUF(dpcf, float, "pcf", pcf.size());
             MC_BUF(dbad2, unsigned char, "bad2", bad.size());
             MC_TRY(hipMemcpyAsync(dpsf, wsh.s.data(), sizeof(float) * psf.size(), hipMemcpyHostToDevice, s));
             MC_TRY(hipMemcpyAsync(dpcf, pcf.data(), sizeof(float) * pcf.size(), hipMemcpyHostToDevice, s));
             MC_TRY(hipMemcpyAsync(dbad2, bad.data(), bad.size(), hipMemcpyHostToDevice, s));
+            // Normalised R2C of `count` real images into spectra at Sf, the
+            // chunks alternating between the streams.
+            auto images_fwd = [&](const float* img, int count) -> int {
+                MC_TRY(fork());
+                for (int f0 = 0; f0 < count; f0 += CH) {
+                    const int nb = std::min(CH, count - f0);
+                    const bool odd = two && ((f0 / CH) & 1);
+                    hipStream_t sk = odd ? c->s2 : s;
+                    cfloat* Tk = odd ? T2 : T;
+                    float* dck = odd ? dcf2 : dcf;
+                    {
+                        KTimer kt(c, "fft_rows_r2c", sk);
+                        MC_TRY(mc_rows_r2c_mod(*pf, img + f0 * rfs, W, rfs, 0, nullptr, Tk, pf->t_elems, nb, scale,
+                                               sk, ff != MC_SPEC_F32 ? dck : nullptr));
+                    }
+                    // a reduced format: new factors from the warped frames' row
+                    // DCs (the inverse above has read this chunk's old ones)
+                    if (ff != MC_SPEC_F32)
+                        MC_TRY(mc_launch_spec_scale(dck, H, nb, gfm + f0, ifm + f0, sk));
+                    {
+                        KTimer kt(c, "fft_cols_fwd", sk);
+                        MC_TRY(mc_cols_fwd(*pf, Tk, pf->t_elems, spec_at(Sf, (long long)f0 * fs, ff), fs, nullptr, 0,
+                                           0, 0, nb, sk, ff, gfm ? gfm + f0 : nullptr));
+                    }
+                }
+                MC_TRY(join());
+                return MC_OK;
+            };
+            // The corrected frames themselves are needed only for the aligned
+            // stack, for weights applied to their spectra, and when their
+            // spectra are to be held in a reduced format.  Otherwise the warp
+            // adds them up, and only the node images of the dose-weighted sums
+            // (and, when the output is binned, the plain sums) are
+            // transformed: fewer than 3/4 of the frames, or it is not worth
+            // the warp's extra accumulators.
+            std::vector<int> cumv(N);
+            std::vector<char> inr(N, 0);
+            for (int i = 0; i < N; i++) {
+                cumv[i] = p->fm_int_size
+                              ? (p->fm_int_start ? p->fm_int_start[i] : i + p->throw0) + p->fm_int_size[i]
+                              : i + 1;
+                const double d = (double)p->fm_dose * cumv[i];
+                inr[i] = !(d < p->sum_range[0]) && !(d > p->sum_range[1]);
+            }
+            bool rising = true;
+            for (int i = 0; i < N; i++) rising = rising && cumv[i] > (i ? cumv[i - 1] : 0);
+            const bool binned = po != pf;
+            const int nplain = 1 + (p->split_sum && !dw ? 2 : 0);
+            bool fused = ff == MC_SPEC_F32 && !p->in_fm_motion && !p->out_stack[0] && rising &&
+                         mc_warp_sums_fit(W, H, keep, wsh.most);
+            SumPlan* sp = nullptr;
+            if (fused) {
+                // a session's movies share their doses: the last plan is kept
+                const double fmax = std::sqrt(0.5) / p->pix_size;
+                const double crit = (0.24499 * std::pow(fmax, -1.6649) + 2.8141) * kvf;
+                const double amax = dw ? 0.5 * p->fm_dose / crit : 0.0;
+                SumPlanKey key{cumv, dws ? inr : std::vector<char>(), dw, p->split_sum != 0, amax};
+                if (!c->sum_plan || !(c->sum_key == key)) {
+                    c->sum_plan.reset(new SumPlan(N, cumv, dw, amax, dws ? &inr : nullptr, p->split_sum != 0,
+                                                  MC_SUM_RANK));
+                    c->sum_key = key;
+                }
+                sp = c->sum_plan.get();
+                fused = 4 * (sp->images + (binned ? nplain : 0)) <= 3 * N;
+            }
+            if (fused) {
+                const int nimg = sp->images + (binned ? nplain : 0);
+                std::vector<int> order, cls, node(N, -1), flags(N, 0);
+                std::vector<float> lam;
+                int im = 0;
+                for (const SumPlan::Class& k : sp->classes) {
+                    const int r = (int)k.nodes.size();
+                    for (int v : {(int)order.size(), (int)k.frames.size(), r, im, k.half}) cls.push_back(v);
+                    for (size_t i = 0; i < k.frames.size(); i++) {
+                        order.push_back(k.frames[i]);
+                        for (int j = 0; j < MC_SUM_RANK; j++)
+                            lam.push_back(j < r ? (float)k.lam[i * r + j] : 0.f);
+                    }
+                    for (int j = 0; j < r; j++) node[k.frames[k.nodes[j]]] = im + j;
+                    im += r;
+                }
+                for (int i = 0; i < N; i++) flags[i] = (inr[i] ? 1 : 0) | (i & 1 ? 2 : 0);
+                // one upload: order, classes, cumulative counts, nodes, flags, coefficients
+                std::vector<int> tab(order);
+                const size_t oc = tab.size();
+                tab.insert(tab.end(), cls.begin(), cls.end());
+                const size_t ou = tab.size();
+                tab.insert(tab.end(), cumv.begin(), cumv.end());
+                tab.insert(tab.end(), node.begin(), node.end());
+                tab.insert(tab.end(), flags.begin(), flags.end());
+                const size_t ol = tab.size();
+                tab.resize(ol + lam.size());
+                std::memcpy(tab.data() + ol, lam.data(), lam.size() * sizeof(float));
+                MC_BUF(dtab, int, "sumtab", tab.size());
+                MC_TRY(hipMemcpyAsync(dtab, tab.data(), sizeof(int) * tab.size(), hipMemcpyHostToDevice, s));
+                MC_BUF(img, float, "Rw", (size_t)std::max(nimg, 1) * W * H);
+                // plain sums: outputs as they are, or images after the nodes'
+                float* pl[3] = {res->sums[0], nplain > 1 ? res->sums[1] : nullptr, nplain > 1 ? res->sums[2] : nullptr};
+                if (binned)
+                    for (int k = 0; k < nplain; k++) pl[k] = img + (sp->images + k) * rfs;
+                {
+                    KTimer kt(c, "local_warp");
+                    MC_TRY(mc_launch_warp_sums(Rr, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any, keep, wsh.most, dtab,
+                                               (const float*)(dtab + ol), dtab + oc, (int)sp->classes.size(), img,
+                                               pl[0], pl[1], pl[2], binned ? 0 : 1, s));
+                }
+                if (nimg) MC_CHECK(images_fwd(img, nimg));
+                MC_TRY(sc.begin(4));
+                if (binned)
+                    for (int k = 0; k < nplain; k++) spec_sums[k] = Sf + (long long)(sp->images + k) * fs;
+                else
+                    for (int k = 0; k < nplain; k++) spec_sums[k] = nullptr;
+                if (dw) {
+                    KTimer kt(c, "dw_sums");
+                    MC_TRY(mc_launch_dw_nodes(Sf, fs, N, g.cx, H, p->pix_size, kvf, p->fm_dose, dtab + ou,
+                                              dtab + ou + N, dtab + ou + 2 * N, dws, p->split_sum, sums + fs, fs, s));
+                }
+            } else {
+            MC_BUF(Rw, float, "Rw", (size_t)N * W * H);
             {
                 KTimer kt(c, "local_warp");
-                const unsigned long long any = bad_any_of(bad.data(), N, P);
-                MC_TRY(mc_launch_local_warp(Rr, Rw, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any,
-                                            mc_warp_keep_max(pcf.data(), any, W, H, P), wsh.most, s));
+                MC_TRY(mc_launch_local_warp(Rr, Rw, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any, keep, wsh.most, s));
             }
-            MC_TRY(fork());
-            for (int f0 = 0; f0 < N; f0 += CH) {
-                const int nb = std::min(CH, N - f0);
-                const bool odd = two && ((f0 / CH) & 1);
-                hipStream_t sk = odd ? c->s2 : s;
-                cfloat* Tk = odd ? T2 : T;
-                float* dck = odd ? dcf2 : dcf;
-                {
-                    KTimer kt(c, "fft_rows_r2c", sk);
-                    MC_TRY(mc_rows_r2c_mod(*pf, Rw + f0 * rfs, W, rfs, 0, nullptr, Tk, pf->t_elems, nb, scale, sk,
-                                           ff != MC_SPEC_F32 ? dck : nullptr));
-                }
-                // a reduced format: new factors from the warped frames' row
-                // DCs (the inverse above has read this chunk's old ones)
-                if (ff != MC_SPEC_F32)
-                    MC_TRY(mc_launch_spec_scale(dck, H, nb, gfm + f0, ifm + f0, sk));
-                {
-                    KTimer kt(c, "fft_cols_fwd", sk);
-                    MC_TRY(mc_cols_fwd(*pf, Tk, pf->t_elems, spec_at(Sf, (long long)f0 * fs, ff), fs, nullptr, 0,
-                                       0, 0, nb, sk, ff, gfm ? gfm + f0 : nullptr));
-                }
-            }
-            MC_TRY(join());
+            MC_CHECK(images_fwd(Rw, N));
             // mGenSums' mMotionDecon (Correct/CCorrectFullShift.cpp:271-320) with
             // the same full shifts (Correct/GCorrectPatchShift.cu:106): the
             // motion weight a second time
@@ -1836,6 +1940,7 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             MC_TRY(mc_launch_dw_sums(Sf, fs, N, g.cx, H, nullptr, nullptr, dw, p->pix_size, kvf,
                                      p->fm_dose, dws, p->sum_range[0], p->sum_range[1], p->split_sum,
                                      sums, fs, s, dcum, ff, ifm));
+            }
         } else {
             // Correct/CCorrectFullShift.cpp:229-309 with the absolute shifts
             MC_TRY(hipMemcpyAsync(gsh, gshift.data(), sizeof(double) * 2 * N, hipMemcpyHostToDevice, s));
@@ -1853,7 +1958,8 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
         // Correct/CCorrectFullShift.cpp:146-185: crop to -FtBin size, C2R, >= 0
         MC_BUF(To, cfloat, "To", (size_t)po->t_elems);
         for (int i = 0; i < nsum; i++) {
-            MC_TRY(mc_cols_inv(*po, sums + (long long)i * fs, fs, g.cx, H, nullptr, To, po->t_elems, 1, s));
+            if (!spec_sums[i]) continue;
+            MC_TRY(mc_cols_inv(*po, spec_sums[i], fs, g.cx, H, nullptr, To, po->t_elems, 1, s));
             MC_TRY(mc_rows_c2r(*po, To, po->t_elems, res->sums[i], g.ow, (long long)g.ow * g.oh, 1, 1, s));
         }
         // -OutStack: Correct/CCorrectFullShift.cpp:336-356 (mCropFrame), every
