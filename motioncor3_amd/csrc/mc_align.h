@@ -101,9 +101,10 @@ hipError_t mc_launch_warp_sums(const float* R, long long pitch, long long fstrid
                                unsigned long long bad_any, int keep_max, float smax, const int* order,
                                const float* lam, const int* cls, int ncls, float* img, float* plain, float* even,
                                float* odd, int clamp, hipStream_t s);
-// Dose-weighted sum spectra from the node images' spectra G.
-hipError_t mc_launch_dw_nodes(const cfloat* G, long long gstride, int N, int cx, int H, double pix, double kvf,
-                              double dose, const int* cum, const int* node, const int* flags, int dws, int split,
+// Dose-weighted sum spectra from the K node images' spectra G; nodes: frame,
+// image and flags (1 in -SumRange, 2 odd) of every node in frame order.
+hipError_t mc_launch_dw_nodes(const cfloat* G, long long gstride, int N, int K, int cx, int H, double pix,
+                              double kvf, double dose, const int* cum, const int* nodes, int dws, int split,
                               cfloat* sums, long long sstride, hipStream_t s);
 // keep_max of the above, from the patch centres on the host
 int mc_warp_keep_max(const float* cen, unsigned long long bad_any, int W, int H, int P);

@@ -1317,12 +1317,14 @@ struct WarpTable {
     unsigned long long* bad;
     unsigned char* klist;  // patch numbers of the kept patches
     int K;
+    int* ord;              // sums: frame number of each row, and its coefficients
+    float4* lam;
 };
 
 // Fill the rows of frames idx(f0) .. idx(f0 + nf - 1).  All threads call it.
 template <class Idx>
 __device__ __forceinline__ void warp_fill(const WarpArgs& a, const WarpTable& t, unsigned long long mask, int f0,
-                                          int nf, Idx idx) {
+                                          int nf, Idx idx, const float* lam) {
     const int nk = __popcll(mask);
     __syncthreads();
     if (threadIdx.x < MC_WARP_FCH) t.bad[threadIdx.x] = 0;
@@ -1339,6 +1341,11 @@ __device__ __forceinline__ void warp_fill(const WarpArgs& a, const WarpTable& t,
             if (a.bad[o]) atomicOr(&t.bad[fi], 1ull << q);
         }
         t.sh[e] = s;
+    }
+    if (t.ord) {
+        if ((int)threadIdx.x < nf) t.ord[threadIdx.x] = idx(f0 + threadIdx.x);
+        for (int e = threadIdx.x; e < nf * MC_SUM_RANK; e += MC_WARP_NT)
+            reinterpret_cast<float*>(t.lam)[e] = lam[f0 * MC_SUM_RANK + e];
     }
     __syncthreads();
 }
@@ -1463,10 +1470,13 @@ struct WarpPixelLds {
 // frames of 2^30 pixels and more (WIDE).
 template <int HOW, bool WIDE, class Px, class Idx, class Use>
 __device__ __forceinline__ void warp_frames(const WarpArgs& a, const Px& px, const WarpTable& t,
-                                            unsigned long long mask, int cnt, Idx idx, Use use) {
+                                            unsigned long long mask, int cnt, Idx idx, const float* lam, Use use) {
     for (int f0 = 0; f0 < cnt; f0 += MC_WARP_FCH) {
         const int nf = min(MC_WARP_FCH, cnt - f0);
-        warp_fill(a, t, mask, f0, nf, idx);
+        warp_fill(a, t, mask, f0, nf, idx, lam);
+        // (a frame number read from LDS is made uniform again: its address and
+        // everything from it is then scalar work)
+        auto frame = [&](int fi) { return t.ord ? __builtin_amdgcn_readfirstlane(t.ord[fi]) : idx(f0 + fi); };
         auto load = [&](int i0, float* d) {
             int so[MC_WARP_U];
             // frames with a bad kept patch sum their own weights; chosen per
@@ -1476,14 +1486,19 @@ __device__ __forceinline__ void warp_frames(const WarpArgs& a, const Px& px, con
             for (int u = 0; u < MC_WARP_U; u++) b |= t.bad[min(i0 + u, nf - 1)];
             if (__builtin_amdgcn_readfirstlane((int)(b | b >> 32))) {
 #pragma unroll
-                for (int u = 0; u < MC_WARP_U; u++) so[u] = px.template source<HOW, true>(a, t, min(i0 + u, nf - 1));
+                for (int u = 0; u < MC_WARP_U; u++) {
+                    const int fi = min(i0 + u, nf - 1);
+                    const unsigned long long f = t.bad[fi];
+                    if (__builtin_amdgcn_readfirstlane((int)(f | f >> 32))) so[u] = px.template source<HOW, true>(a, t, fi);
+                    else so[u] = px.template source<HOW, false>(a, t, fi);
+                }
             } else {
 #pragma unroll
                 for (int u = 0; u < MC_WARP_U; u++) so[u] = px.template source<HOW, false>(a, t, min(i0 + u, nf - 1));
             }
 #pragma unroll
             for (int u = 0; u < MC_WARP_U; u++) {
-                const float* __restrict__ fr = a.R + (long long)idx(f0 + min(i0 + u, nf - 1)) * a.fstride;
+                const float* __restrict__ fr = a.R + (long long)frame(min(i0 + u, nf - 1)) * a.fstride;
                 if constexpr (WIDE) d[u] = fr[so[u]];
                 else d[u] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(fr) + ((unsigned)so[u] << 2));
             }
@@ -1493,7 +1508,7 @@ __device__ __forceinline__ void warp_frames(const WarpArgs& a, const Px& px, con
         for (int i0 = 0; i0 < nf; i0 += MC_WARP_U) {
             float vn[MC_WARP_U];
             if (i0 + MC_WARP_U < nf) load(i0 + MC_WARP_U, vn);
-            use(f0 + i0, min(MC_WARP_U, nf - i0), v);
+            use(f0, i0, min(MC_WARP_U, nf - i0), v);
 #pragma unroll
             for (int u = 0; u < MC_WARP_U; u++) v[u] = vn[u];
         }
@@ -1506,7 +1521,9 @@ __device__ __forceinline__ void warp_store(const WarpArgs& a, const WarpTable& t
     Px px;
     px.init(a, mask, x, y, lds);
     float* __restrict__ out = a.Rp + (long long)y * a.pitch + x;
-    warp_frames<HOW, WIDE>(a, px, t, mask, a.N, [](int i) { return i; }, [&](int i0, int n, const float* v) {
+    warp_frames<HOW, WIDE>(a, px, t, mask, a.N, [](int i) { return i; }, nullptr,
+                           [&](int f0, int fi, int n, const float* v) {
+        const int i0 = f0 + fi;
         if (n == MC_WARP_U) {
             // unconditional stores: a conditional one sits in a block of its
             // own, where the compiler waits for every outstanding access
@@ -1540,7 +1557,7 @@ __global__ __launch_bounds__(MC_WARP_NT, CLASS == 0 ? 4 : 2) void k_local_warp(W
     __shared__ float4 tab[MC_WARP_FCH * KMAX / 2];
     __shared__ unsigned long long bad[MC_WARP_FCH];
     __shared__ unsigned char klist[MC_WARP_MAXP];
-    WarpTable t{reinterpret_cast<float2*>(tab), bad, klist, 0};
+    WarpTable t{reinterpret_cast<float2*>(tab), bad, klist, 0, nullptr, nullptr};
     const float m = a.smax + 1.f;
     const bool inner = x0 >= m && y0 >= m && x0 + 63 < a.W - m && y0 + 3 < a.H - m;
 #define MC_WK(KK)                                                                                    \
@@ -1571,8 +1588,11 @@ __global__ __launch_bounds__(MC_WARP_NT, CLASS == 0 ? 4 : 2) void k_local_warp(W
 // for a few node frames j to below FP32 rounding (SumPlan in mc_host.cpp),
 // and sum_i q^c_i F_i = sum_j q^c_j FFT(sum_i lam_ij frame_i): the transforms
 // run over one image per node, 16 instead of 50 at 1 e-/px and frame.
-// Bound by the gathers (4 B per pixel and frame) and the warp's vector work;
-// the accumulators add MC_SUM_RANK FMAs per pixel and frame.
+// Bound by the warp's vector work (88% busy), to which the accumulators add
+// MC_SUM_RANK FMAs per pixel and frame: 2.8 ms at 5760 x 4092, 50 frames, 25
+// patches, where the storing warp (2.9), 50 transforms (4.7) and k_dw_sums
+// (1.1) took 8.7.  Class tables read through vector loads kept the frame
+// addresses in vector registers: 3.6 ms.
 struct WarpSumArgs {
     WarpArgs w;
     const int* order;     // frames, class by class
@@ -1594,22 +1614,36 @@ __device__ __forceinline__ void warp_sum(const WarpSumArgs& s, const WarpTable& 
     const long long o = (long long)y * a.pitch + x;
     float total = 0.f;
     for (int c = 0; c < s.ncls; c++) {
-        const int* __restrict__ cl = s.cls + 5 * c;
-        const int first = cl[0], nodes = cl[2];
-        const int* __restrict__ order = s.order + first;
-        const float* __restrict__ lam = s.lam + first * MC_SUM_RANK;
+        int cl[5];
+#pragma unroll
+        for (int k = 0; k < 5; k++) cl[k] = __builtin_amdgcn_readfirstlane(s.cls[5 * c + k]);
+        const int nodes = cl[2];
+        const int* order = s.order + cl[0];
         float acc[MC_SUM_RANK], sum = 0.f;
 #pragma unroll
         for (int j = 0; j < MC_SUM_RANK; j++) acc[j] = 0.f;
-        warp_frames<HOW, false>(a, px, t, mask, cl[1], [&](int i) { return order[i]; },
-                                [&](int i0, int n, const float* v) {
+        auto add = [&](int fi, float v) {
+            sum += v;
+            const float4 l0 = t.lam[2 * fi], l1 = t.lam[2 * fi + 1];
+            acc[0] = fmaf(l0.x, v, acc[0]);
+            acc[1] = fmaf(l0.y, v, acc[1]);
+            acc[2] = fmaf(l0.z, v, acc[2]);
+            acc[3] = fmaf(l0.w, v, acc[3]);
+            acc[4] = fmaf(l1.x, v, acc[4]);
+            acc[5] = fmaf(l1.y, v, acc[5]);
+            acc[6] = fmaf(l1.z, v, acc[6]);
+            acc[7] = fmaf(l1.w, v, acc[7]);
+        };
+        static_assert(MC_SUM_RANK == 8, "two float4 of coefficients per frame");
+        warp_frames<HOW, false>(a, px, t, mask, cl[1], [&](int i) { return order[i]; }, s.lam + cl[0] * MC_SUM_RANK,
+                                [&](int, int fi, int n, const float* v) {
+            if (n == MC_WARP_U) {
 #pragma unroll
-            for (int u = 0; u < MC_WARP_U; u++) {
-                if (u >= n) break;
-                sum += v[u];
-                if (nodes)
+                for (int u = 0; u < MC_WARP_U; u++) add(fi + u, v[u]);
+            } else {
 #pragma unroll
-                    for (int j = 0; j < MC_SUM_RANK; j++) acc[j] = fmaf(lam[(i0 + u) * MC_SUM_RANK + j], v[u], acc[j]);
+                for (int u = 0; u < MC_WARP_U; u++)
+                    if (u < n) add(fi + u, v[u]);
             }
         });
         float* __restrict__ im = s.img + cl[3] * a.fstride + o;
@@ -1633,7 +1667,9 @@ __global__ __launch_bounds__(MC_WARP_NT, CLASS == 0 ? 4 : 2) void k_warp_sums(Wa
     __shared__ float4 tab[MC_WARP_FCH * (CLASS == 0 ? 16 : MC_WARP_KREG) / 2];
     __shared__ unsigned long long bad[MC_WARP_FCH];
     __shared__ unsigned char klist[MC_WARP_MAXP];
-    WarpTable t{reinterpret_cast<float2*>(tab), bad, klist, 0};
+    __shared__ int ord[MC_WARP_FCH];
+    __shared__ float4 lam[MC_WARP_FCH * MC_SUM_RANK / 4];
+    WarpTable t{reinterpret_cast<float2*>(tab), bad, klist, 0, ord, lam};
     const float m = a.smax + 1.f;
     const bool inner = x0 >= m && y0 >= m && x0 + 63 < a.W - m && y0 + 3 < a.H - m;
 #define MC_WK(KK)                                                             \
@@ -1747,17 +1783,20 @@ __global__ __launch_bounds__(256) void k_dw_sums(DwArgs a) {
     }
 }
 
-// The dose-weighted sums of k_dw_sums from node images (k_warp_sums): node
-// frame i's spectrum is image node[i], its weight the frame's own.  flags[i]:
-// bit 0 in -SumRange, bit 1 odd.
+// The dose-weighted sums of k_dw_sums from node images (k_warp_sums): node k,
+// in frame order, is frame nodes[3k]'s weight on image nodes[3k + 1]; its bits
+// nodes[3k + 2]: 1 in -SumRange, 2 an odd frame.  One pass over the frames
+// forms the powers and the normaliser (relative to the first frame's weight,
+// so that they stay in FP32's range), the images' values four loads ahead:
+// 5760 x 4092, 50 frames, 16 nodes 0.43 ms, against 0.58 with two passes and a load
+// at a time.
 struct DwNodeArgs {
     const cfloat* G;
     long long gstride;
-    int N, cx, H;
+    int N, K, cx, H;
     double pix, kvf, dose;
     const int* cum;      // raw frames counted into frame i's dose
-    const int* node;     // image of frame i, or -1
-    const int* flags;
+    const int* nodes;
     int dws, split;
     cfloat* sums;        // _DW, then _DWS, even and odd as asked for
     long long sstride;
@@ -1767,40 +1806,52 @@ __global__ __launch_bounds__(256) void k_dw_nodes(DwNodeArgs a) {
     const int kx = blockIdx.y;
     const int y = blockIdx.x * blockDim.x + threadIdx.x;
     if (y >= a.H) return;
-    const long long q = (long long)kx * a.H + y;
-    double qd = 1.0, inv_ws = 1.0;
-    if (kx != 0 || y != 0) {
-        qd = crit_q(kx, y, a.cx, a.H, a.pix, a.kvf, a.dose);
-        double w = 1.0, s = 0.0;
-        int prev = 0;
-        for (int i = 0; i < a.N; i++) {
-            const int c = a.cum[i];
-            for (int k = prev; k < c; k++) w *= qd;
-            prev = c;
+    const unsigned q = (unsigned)kx * a.H + y;
+    const bool dc = kx == 0 && y == 0;
+    const double qd = dc ? 1.0 : crit_q(kx, y, a.cx, a.H, a.pix, a.kvf, a.dose);
+    cfloat s1 = cmk(0.f, 0.f), s2 = s1, so = s1, se = s1;
+    double w = 1.0, s = 0.0;
+    int i = 0;
+    // weights up to and including frame f
+    auto advance = [&](int f) {
+        for (; i <= f; i++) {
+            if (i > 0)
+                for (int k = a.cum[i - 1]; k < a.cum[i]; k++) w *= qd;
             s += w * w;
         }
-        inv_ws = 1.0 / sqrt(s);
+    };
+    constexpr int U = 4;
+    cfloat g[U];
+    auto load = [&](int k0, cfloat* d) {
+#pragma unroll
+        for (int u = 0; u < U; u++) d[u] = (a.G + (long long)a.nodes[3 * min(k0 + u, a.K - 1) + 1] * a.gstride)[q];
+    };
+    load(0, g);
+    for (int k0 = 0; k0 < a.K; k0 += U) {
+        cfloat gn[U];
+        if (k0 + U < a.K) load(k0 + U, gn);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (k0 + u >= a.K) break;
+            advance(a.nodes[3 * (k0 + u)]);
+            const int fl = a.nodes[3 * (k0 + u) + 2];
+            const cfloat v = cscale(g[u], (float)w);
+            s1 = cadd(s1, v);
+            if (fl & 1) s2 = cadd(s2, v);
+            if (fl & 2) so = cadd(so, v);
+            else se = cadd(se, v);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) g[u] = gn[u];
     }
-    cfloat s1 = cmk(0.f, 0.f), s2 = s1, so = s1, se = s1;
-    double w = 1.0;
-    int prev = 0;
-    for (int i = 0; i < a.N; i++) {
-        const int c = a.cum[i], nd = a.node[i], fl = a.flags[i];
-        for (int k = prev; k < c; k++) w *= qd;
-        prev = c;
-        if (nd < 0) continue;
-        const cfloat v = cscale(a.G[(long long)nd * a.gstride + q], (float)(w * inv_ws));
-        s1 = cadd(s1, v);
-        if (fl & 1) s2 = cadd(s2, v);
-        if (fl & 2) so = cadd(so, v);
-        else se = cadd(se, v);
-    }
+    advance(a.N - 1);
+    const float inv = dc ? 1.f : (float)(1.0 / sqrt(s));
     int ns = 0;
-    a.sums[(long long)(ns++) * a.sstride + q] = s1;
-    if (a.dws) a.sums[(long long)(ns++) * a.sstride + q] = s2;
+    (a.sums + (ns++) * a.sstride)[q] = cscale(s1, inv);
+    if (a.dws) (a.sums + (ns++) * a.sstride)[q] = cscale(s2, inv);
     if (a.split) {
-        a.sums[(long long)ns * a.sstride + q] = se;
-        a.sums[(long long)(ns + 1) * a.sstride + q] = so;
+        (a.sums + ns * a.sstride)[q] = cscale(se, inv);
+        (a.sums + (ns + 1) * a.sstride)[q] = cscale(so, inv);
     }
 }
 
@@ -2149,10 +2200,11 @@ bool mc_warp_sums_fit(long long pitch, int H, int keep_max, float smax) {
     return pitch * H < (1LL << 30) && smax >= 0 && warp_class(keep_max) <= 1;
 }
 
-hipError_t mc_launch_dw_nodes(const cfloat* G, long long gstride, int N, int cx, int H, double pix, double kvf,
-                              double dose, const int* cum, const int* node, const int* flags, int dws, int split,
+hipError_t mc_launch_dw_nodes(const cfloat* G, long long gstride, int N, int K, int cx, int H, double pix,
+                              double kvf, double dose, const int* cum, const int* nodes, int dws, int split,
                               cfloat* sums, long long sstride, hipStream_t s) {
-    DwNodeArgs a{G, gstride, N, cx, H, pix, kvf, dose, cum, node, flags, dws, split, sums, sstride};
+    if (N < 1 || K < 1) return hipErrorInvalidValue;
+    DwNodeArgs a{G, gstride, N, K, cx, H, pix, kvf, dose, cum, nodes, dws, split, sums, sstride};
     hipLaunchKernelGGL(k_dw_nodes, dim3(mc_div_up(H, 256), cx), dim3(256), 0, s, a);
     return hipGetLastError();
 }

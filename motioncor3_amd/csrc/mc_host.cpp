@@ -1874,7 +1874,7 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             }
             if (fused) {
                 const int nimg = sp->images + (binned ? nplain : 0);
-                std::vector<int> order, cls, node(N, -1), flags(N, 0);
+                std::vector<int> order, cls, node(N, -1), nodes;
                 std::vector<float> lam;
                 int im = 0;
                 for (const SumPlan::Class& k : sp->classes) {
@@ -1888,15 +1888,16 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
                     for (int j = 0; j < r; j++) node[k.frames[k.nodes[j]]] = im + j;
                     im += r;
                 }
-                for (int i = 0; i < N; i++) flags[i] = (inr[i] ? 1 : 0) | (i & 1 ? 2 : 0);
-                // one upload: order, classes, cumulative counts, nodes, flags, coefficients
+                for (int i = 0; i < N; i++)
+                    if (node[i] >= 0)
+                        for (int v : {i, node[i], (inr[i] ? 1 : 0) | (i & 1 ? 2 : 0)}) nodes.push_back(v);
+                // one upload: order, classes, cumulative counts, nodes, coefficients
                 std::vector<int> tab(order);
                 const size_t oc = tab.size();
                 tab.insert(tab.end(), cls.begin(), cls.end());
                 const size_t ou = tab.size();
                 tab.insert(tab.end(), cumv.begin(), cumv.end());
-                tab.insert(tab.end(), node.begin(), node.end());
-                tab.insert(tab.end(), flags.begin(), flags.end());
+                tab.insert(tab.end(), nodes.begin(), nodes.end());
                 const size_t ol = tab.size();
                 tab.resize(ol + lam.size());
                 std::memcpy(tab.data() + ol, lam.data(), lam.size() * sizeof(float));
@@ -1921,8 +1922,8 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
                     for (int k = 0; k < nplain; k++) spec_sums[k] = nullptr;
                 if (dw) {
                     KTimer kt(c, "dw_sums");
-                    MC_TRY(mc_launch_dw_nodes(Sf, fs, N, g.cx, H, p->pix_size, kvf, p->fm_dose, dtab + ou,
-                                              dtab + ou + N, dtab + ou + 2 * N, dws, p->split_sum, sums + fs, fs, s));
+                    MC_TRY(mc_launch_dw_nodes(Sf, fs, N, sp->images, g.cx, H, p->pix_size, kvf, p->fm_dose,
+                                              dtab + ou, dtab + ou + N, dws, p->split_sum, sums + fs, fs, s));
                 }
             } else {
             MC_BUF(Rw, float, "Rw", (size_t)N * W * H);

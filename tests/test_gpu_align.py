@@ -292,3 +292,44 @@ def test_frame_weights_do_not_race_the_patch_preparation(ctx):
         assert np.array_equal(one["global_shift"], two["global_shift"]), rep
         for a, b in zip(one["sums"], two["sums"]):
             assert np.array_equal(a.numpy(), b.numpy()), rep
+
+
+def _replay(N, P, W, H, n, seed):
+    rng = np.random.default_rng(seed)
+    cen = np.array([[(i % n + 0.5) * W / n, (i // n + 0.5) * H / n] for i in range(P)], np.float32)
+    return dict(replay_global=np.round(np.cumsum(rng.normal(0, 0.4, (N, 2)), 0), 2).astype(np.float32),
+                replay_patch=rng.normal(0, 2.0, (N, P, 2)).astype(np.float32), replay_centers=cen,
+                replay_bad=(rng.random((N, P)) < 0.05).astype(np.uint8))
+
+
+# frames per gather group and table, doses from one class of nodes to several
+# and to one node per frame, sums with and without ranges, halves and binning,
+# integrated frames, more patches than one register class
+@pytest.mark.parametrize("N,n,kw", [
+    (9, 2, dict()), (33, 3, dict(split_sum=1)), (33, 3, dict(split_sum=1, ft_bin=2.0)),
+    (24, 3, dict(fm_dose=0.5)), (24, 3, dict(fm_dose=0.5, ft_bin=1.5)), (41, 3, dict(fm_dose=1.3)),
+    (41, 3, dict(fm_dose=1.3, sum_range=(-1.0, 0.0))), (66, 2, dict(fm_dose=0.4, split_sum=1)),
+    (24, 3, dict(fm_dose=6.0)), (24, 7, dict(fm_dose=0.5)), (20, 3, dict(fm_dose=0.3, kv=120, ints=True)),
+])
+def test_sums_without_stored_frames_match_stored(ctx, N, n, kw):
+    """Patch mode's sums formed while warping, with dose weights from node
+    images, against the path that stores every corrected frame (asking for the
+    aligned stack takes it) with the same shifts.  The weights differ by at
+    most 3.3e-8 of their normaliser, the transforms' roundings by a few 1e-7:
+    under 1e-6 of the sums' norm."""
+    print("fused sums", N, n, kw, flush=True)
+    W, H, P = 330, 258, n * n
+    kw = dict(kw)
+    if kw.pop("ints", False):
+        size = np.array([1 + i % 3 for i in range(N)], np.int32)
+        kw.update(fm_int_start=np.concatenate([[0], np.cumsum(size)[:-1]]).astype(np.int32), fm_int_size=size)
+    rng = np.random.default_rng(N + n)
+    frames = ctx.upload(rng.poisson(1.0, (N, H, W)).astype(np.float32))
+    rep = _replay(N, P, W, H, n, N)
+    base = dict(patch=(n, n), pix_size=0.9, **kw)
+    out = ctx.align_movie(frames, L.default_params(**base), **rep)
+    ref = ctx.align_movie(frames, L.default_params(out_stack=(1, 1), **base), **rep)
+    assert out["num_sums"] == ref["num_sums"]
+    for a, b in zip(out["sums"], ref["sums"]):
+        a, b = a.numpy(), b.numpy()
+        assert np.linalg.norm(a - b) < 1e-6 * np.linalg.norm(b)
