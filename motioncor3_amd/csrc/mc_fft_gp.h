@@ -66,7 +66,7 @@ struct GpTables {              // device memory of a plan (owned by the Fft2D)
     GpPlan* plan = nullptr;
 };
 
-// A plan for length n, or false when it has none (too long for LDS).
+// A plan for length n, or false and P->n = 0 when it has none (too long for LDS).
 bool gp_plan(int n, GpPlan* P, GpTables* T);
 void gp_free(GpTables* T);
 int mc_fft_gp_init();

@@ -521,7 +521,7 @@ bool gp_attr(F* f) {
 
 }  // namespace
 
-bool gp_plan(int n, GpPlan* P, GpTables* T) {
+static bool gp_build(int n, GpPlan* P, GpTables* T) {
     static const std::vector<int> plain = {
 #define X(R) R,
         MC_GP_RADICES(X)
@@ -656,6 +656,12 @@ bool gp_plan(int n, GpPlan* P, GpTables* T) {
     }
     P->dev = T->plan;
     return true;
+}
+
+bool gp_plan(int n, GpPlan* P, GpTables* T) {
+    if (gp_build(n, P, T)) return true;
+    *P = GpPlan();  // n = 0: callers take the stage kernels
+    return false;
 }
 
 void gp_free(GpTables* T) {

@@ -243,6 +243,20 @@ def test_run_time_radix_passes(ctx, W, H):
     assert np.array_equal(got[1:].reshape(B, H, pitch)[:, :, :W], dense)
 
 
+@pytest.mark.parametrize("W,H", [(17304, 12), (24, 8652)])
+def test_lengths_past_the_run_time_plans(ctx, W, H):
+    """8652 = 84 * 103: its chirp convolution of 17303 points does not fit
+    LDS, so the stage kernels take it.  Their stage of 103 sums 103 products:
+    at most 103 roundings of 6e-8 on top of the other stages', typically their
+    root; 2e-6."""
+    print("past the run-time plans", W, H, flush=True)
+    x = np.random.default_rng(3).standard_normal((2, H, W)).astype(np.float32)
+    ref = np.fft.rfft2(x.astype(np.float64)).transpose(0, 2, 1)
+    assert _rel(ctx.rfft2(ctx.upload(x)).numpy(), ref) < 2e-6
+    back = ctx.irfft2(ctx.upload(ref.astype(np.complex64)), W).numpy()
+    assert _rel(back, x.astype(np.float64) * (W * H)) < 2e-6
+
+
 @pytest.mark.parametrize("W,H,ft_bin", [(1000, 600, 2.0), (740, 820, 1.5), (3838, 3710, 2.0)])
 def test_run_time_radix_crop(ctx, W, H, ft_bin):
     """The Fourier crop in the inverse column pass (output sums at the -FtBin
