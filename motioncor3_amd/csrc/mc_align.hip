@@ -1236,10 +1236,10 @@ struct WarpArgs {
     long long pitch, fstride;
     int W, H, N, P;
     const float* cen;
-    const float* sh;             // N x P x 2, zero where bad
+    const float* sh;             // N x P x 2
     const unsigned char* bad;    // N x P
     unsigned long long bad_any;  // bit p: patch p is bad in some frame
-    float smax;                  // largest |shift| in sh; below 0: not finite or absurd
+    float smax;                  // bound on the shifts of good patches; below 0: none (not finite, absurd)
 };
 
 // a / b with r = 1 / b correctly rounded: the remainder of the approximate
@@ -1337,8 +1337,8 @@ __device__ __forceinline__ void warp_fill(const WarpArgs& a, const WarpTable& t,
         if (q < nk) {
             const int p = t.klist[q];
             const long long o = (long long)idx(f0 + fi) * a.P + p;
-            s = reinterpret_cast<const float2*>(a.sh)[o];
             if (a.bad[o]) atomicOr(&t.bad[fi], 1ull << q);
+            else s = reinterpret_cast<const float2*>(a.sh)[o];
         }
         t.sh[e] = s;
     }

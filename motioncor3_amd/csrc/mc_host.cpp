@@ -324,22 +324,26 @@ unsigned long long bad_any_of(const unsigned char* bad, int N, int P) {
     return m;
 }
 
-// The local warp's view of an N x P x 2 shift table: zero where a patch is
-// bad, and its largest magnitude (-1 when a shift is not finite or above 1e5).
-struct WarpShifts {
-    std::vector<float> s;
+// Largest magnitude of an N x P x 2 shift table outside the bad patches, the
+// bound the local warp takes for its tiles (-1 when a shift is not finite or
+// above 1e5).
+float warp_shift_max(const float* shifts, const unsigned char* bad, int N, int P) {
     float most = 0.f;
-    WarpShifts(const float* shifts, const unsigned char* bad, int N, int P)
-        : s(shifts, shifts + 2 * (size_t)N * P) {
-        bool safe = true;
-        for (size_t e = 0; e < s.size(); e++) {
-            if (bad && bad[e / 2]) s[e] = 0.f;
-            if (!(std::fabs(s[e]) <= 1e5f)) safe = false;
-            most = std::max(most, std::fabs(s[e]));
-        }
-        if (!safe) most = -1.f;
+    for (size_t e = 0; e < 2 * (size_t)N * P; e++) {
+        if (bad && bad[e / 2]) continue;
+        if (!(std::fabs(shifts[e]) <= 1e5f)) return -1.f;
+        most = std::max(most, std::fabs(shifts[e]));
     }
-};
+    return most;
+}
+
+// The same for a launch: a captured one reads its tables again at each replay,
+// when they may hold other shifts, so it takes no bound from these.
+float warp_launch_max(const float* shifts, const unsigned char* bad, int N, int P, hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return -1.f;
+    return warp_shift_max(shifts, bad, N, P);
+}
 
 // ---------------------------------------------------------------------------
 // geometry: CBufferPool.cpp:185-262, Align/CAlignBase.cpp:41-47
@@ -1798,13 +1802,13 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             std::vector<float> psf(ps.size()), pcf(pc.size());
             for (size_t i = 0; i < ps.size(); i++) psf[i] = (float)ps[i];
             for (size_t i = 0; i < pc.size(); i++) pcf[i] = (float)pc[i];
-            const WarpShifts wsh(psf.data(), bad.data(), N, P);
+            const float most = warp_shift_max(psf.data(), bad.data(), N, P);
             const unsigned long long any = bad_any_of(bad.data(), N, P);
             const int keep = mc_warp_keep_max(pcf.data(), any, W, H, P);
             MC_BUF(dpsf, float, "psf", psf.size());
             MC_BUF(dpcf, float, "pcf", pcf.size());
             MC_BUF(dbad2, unsigned char, "bad2", bad.size());
-            MC_TRY(hipMemcpyAsync(dpsf, wsh.s.data(), sizeof(float) * psf.size(), hipMemcpyHostToDevice, s));
+            MC_TRY(hipMemcpyAsync(dpsf, psf.data(), sizeof(float) * psf.size(), hipMemcpyHostToDevice, s));
             MC_TRY(hipMemcpyAsync(dpcf, pcf.data(), sizeof(float) * pcf.size(), hipMemcpyHostToDevice, s));
             MC_TRY(hipMemcpyAsync(dbad2, bad.data(), bad.size(), hipMemcpyHostToDevice, s));
             // Normalised R2C of `count` real images into spectra at Sf, the
@@ -1856,7 +1860,7 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             const bool binned = po != pf;
             const int nplain = 1 + (p->split_sum && !dw ? 2 : 0);
             bool fused = ff == MC_SPEC_F32 && !p->in_fm_motion && !p->out_stack[0] && rising &&
-                         mc_warp_sums_fit(W, H, keep, wsh.most);
+                         mc_warp_sums_fit(W, H, keep, most);
             SumPlan* sp = nullptr;
             if (fused) {
                 // a session's movies share their doses: the last plan is kept
@@ -1910,7 +1914,7 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
                     for (int k = 0; k < nplain; k++) pl[k] = img + (sp->images + k) * rfs;
                 {
                     KTimer kt(c, "local_warp");
-                    MC_TRY(mc_launch_warp_sums(Rr, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any, keep, wsh.most, dtab,
+                    MC_TRY(mc_launch_warp_sums(Rr, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any, keep, most, dtab,
                                                (const float*)(dtab + ol), dtab + oc, (int)sp->classes.size(), img,
                                                pl[0], pl[1], pl[2], binned ? 0 : 1, s));
                 }
@@ -1929,7 +1933,7 @@ int align_batch(mc_ctx* c, const mc_params* const* pp_, const mc_movie* const* m
             MC_BUF(Rw, float, "Rw", (size_t)N * W * H);
             {
                 KTimer kt(c, "local_warp");
-                MC_TRY(mc_launch_local_warp(Rr, Rw, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any, keep, wsh.most, s));
+                MC_TRY(mc_launch_local_warp(Rr, Rw, W, rfs, W, H, N, P, dpcf, dpsf, dbad2, any, keep, most, s));
             }
             MC_CHECK(images_fwd(Rw, N));
             // mGenSums' mMotionDecon (Correct/CCorrectFullShift.cpp:271-320) with
@@ -2528,13 +2532,13 @@ int mc_local_warp(mc_ctx* c, const float* in, float* out, int W, int H, int N, i
     MC_BUF(ds, float, "api_ws", (size_t)2 * N * P);
     MC_BUF(db, unsigned char, "api_wb", (size_t)N * P);
     MC_TRY(hipMemcpyAsync(dc, centers, sizeof(float) * 2 * P, hipMemcpyHostToDevice, c->stream));
-    const WarpShifts sh(shifts, bad, N, P);
-    MC_TRY(hipMemcpyAsync(ds, sh.s.data(), sizeof(float) * 2 * N * P, hipMemcpyHostToDevice, c->stream));
+    MC_TRY(hipMemcpyAsync(ds, shifts, sizeof(float) * 2 * N * P, hipMemcpyHostToDevice, c->stream));
     if (bad) MC_TRY(hipMemcpyAsync(db, bad, (size_t)N * P, hipMemcpyHostToDevice, c->stream));
     else MC_TRY(hipMemsetAsync(db, 0, (size_t)N * P, c->stream));
     const unsigned long long any = bad_any_of(bad, N, P);
     MC_TRY(mc_launch_local_warp(in, out, W, (long long)W * H, W, H, N, P, dc, ds, db, any,
-                                mc_warp_keep_max(centers, any, W, H, P), sh.most, c->stream));
+                                mc_warp_keep_max(centers, any, W, H, P),
+                                warp_launch_max(shifts, bad, N, P, c->stream), c->stream));
     return MC_OK;
 }
 
@@ -2565,14 +2569,14 @@ int mc_local_warp_noalloc(mc_ctx* c, const float* in, float* out, int W, int H, 
     float* ds = (float*)(c->scratch + os);
     unsigned char* db = c->scratch + ob;
     MC_TRY(hipMemcpyAsync(dc, centers, sizeof(float) * 2 * P, hipMemcpyHostToDevice, c->stream));
-    const WarpShifts sh(shifts, bad, N, P);
-    MC_TRY(hipMemcpyAsync(ds, sh.s.data(), sizeof(float) * 2 * (size_t)N * P, hipMemcpyHostToDevice, c->stream));
+    MC_TRY(hipMemcpyAsync(ds, shifts, sizeof(float) * 2 * (size_t)N * P, hipMemcpyHostToDevice, c->stream));
     // the previous call's flags are still there: write or clear all of them
     if (bad) MC_TRY(hipMemcpyAsync(db, bad, (size_t)N * P, hipMemcpyHostToDevice, c->stream));
     else MC_TRY(mc_launch_fill_u8(db, (long long)N * P, 0, c->stream));
     const unsigned long long any = bad_any_of(bad, N, P);
     MC_TRY(mc_launch_local_warp(in, out, W, (long long)W * H, W, H, N, P, dc, ds, db, any,
-                                mc_warp_keep_max(centers, any, W, H, P), sh.most, c->stream));
+                                mc_warp_keep_max(centers, any, W, H, P),
+                                warp_launch_max(shifts, bad, N, P, c->stream), c->stream));
     return MC_OK;
 }
 

@@ -62,3 +62,40 @@ def test_noalloc_warp_rejects_tables_beyond_its_scratch(ctx):
     rc, _ = _noalloc(ctx, frames, cen, sh, None)
     assert rc == L.MC_E_ARG
     assert b"scratch" in ctx.lib.mc_last_error(ctx.ptr)
+
+
+def test_noalloc_warp_captured_reads_its_tables_at_replay(ctx):
+    """A captured call copies the caller's shift table at every replay: with
+    other values in it, larger and non-zero under a bad flag, each replay gives
+    what a direct call with them gives."""
+    hip = C.CDLL("libamdhip64.so.7")
+    stream, graph, run = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+    own = L.Context(0, stream.value)
+    rng = np.random.default_rng(5)
+    frames, cen, sh, bad = _case(rng, 5, 96, 128, 9, True)
+    d, out = own.upload(frames), own.empty(frames.shape, np.float32)
+    fp, bp = C.POINTER(C.c_float), bad.ctypes.data_as(C.POINTER(C.c_ubyte))
+
+    def call():
+        return own.lib.mc_local_warp_noalloc(own.ptr, d.vp(), out.vp(), 128, 96, 5, 9, cen.ctypes.data_as(fp),
+                                             sh.ctypes.data_as(fp), bp)
+
+    assert call() == L.MC_OK
+    own.sync()
+    print("capture", flush=True)
+    assert hip.hipStreamBeginCapture(stream, 2) == 0
+    rc = call()
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and rc == L.MC_OK
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for k in range(3):
+        sh[:] = rng.uniform(-20 * (k + 1), 20 * (k + 1), sh.shape)
+        print("replay", k, flush=True)
+        assert hip.hipGraphLaunch(run, stream) == 0
+        own.sync()
+        assert np.array_equal(out.numpy(), own.local_warp(d, cen, sh, bad).numpy()), k
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    d.free()
+    out.free()
+    own.close()
+    assert hip.hipStreamDestroy(stream) == 0
