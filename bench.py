@@ -28,34 +28,40 @@ sys.path.insert(0, ROOT)
 METRIC = "movies/s @5760x4092x50 frames, 5x5 patches; shift RMS err vs FP64 (px)"
 W, H, N = 5760, 4092, 50
 PEAK_HBM_GBS = 8000.0
+# Node images of the dose-weighted sums in this workload (50 frames of
+# 1 e/A^2, sum range 3-25: classes of 23, 2 and 25 frames on 7, 2 and 7
+# nodes).  With FP32 frame spectra the second forward pass transforms these,
+# not the corrected frames.
+SUM_IMAGES = 16
 
 
-def algorithmic_bytes(kernel, g, launches):
+def algorithmic_bytes(kernel, g, launches, images):
     """Compulsory HBM bytes of one launch of `kernel` in this workload:
     each stage reads its inputs once and writes its outputs once; `launches`
     is the kernel class's launch count per movie (the forward classes run in
     the forward and local-correction passes, the inverse ones in the second
-    only)."""
+    only); the second forward pass transforms `images` images (N when the
+    corrected frames themselves are transformed)."""
     cx, xcx = W // 2 + 1, g["xcf"][0] // 2 + 1
     S_f = 8.0 * cx * H                         # full half spectrum
     R_f = 4.0 * W * H                          # full real frame
     S_x = 8.0 * xcx * g["xcf"][1]              # xcf half spectrum
     if kernel == "fft_cols_fwd":               # T -> S (+ xcf crop in the first pass)
-        return (N * 2 * S_f + N * S_x + N * 2 * S_f) / launches
+        return (N * 2 * S_f + N * S_x + images * 2 * S_f) / launches
     if kernel == "fft_rows_r2c":               # real -> T
-        return (2 * N * (R_f + S_f)) / launches
+        return ((N + images) * (R_f + S_f)) / launches
     if kernel == "fft_cols_inv":               # S -> T
         return N * 2 * S_f / launches
     if kernel == "fft_rows_c2r":               # T -> real
         return N * (S_f + R_f) / launches
-    if kernel == "local_warp":                 # all frames, read + write
-        return N * 2 * R_f
-    if kernel == "dw_sums":                    # N spectra in, 3 sums out
-        return N * S_f + 3 * S_f
+    if kernel == "local_warp":                 # frames in, frames or images and plain sum out
+        return N * 2 * R_f if images == N else (N + images + 1) * R_f
+    if kernel == "dw_sums":                    # spectra in, sums (two of them weighted) out
+        return images * S_f + (3 if images == N else 2) * S_f
     raise ValueError(kernel)
 
 
-def path_bytes(g, iters_global, iters_patch, nsum, P=25):
+def path_bytes(g, iters_global, iters_patch, nsum, images, P=25):
     """Compulsory HBM bytes of one movie through the whole path: every stage
     reads its inputs once and writes its outputs once (FFT = one read + one
     write), adjacent elementwise stages fused."""
@@ -67,9 +73,11 @@ def path_bytes(g, iters_global, iters_patch, nsum, P=25):
     S_p, R_p = 8.0 * (pw // 2 + 1) * ph, 4.0 * pw * ph
     b = N * (R_f + S_f) + 2 * N * S_x + iters_global * (2 * N + 2) * S_x
     b += ((N + 1) * S_x + N * (S_x + R_x) + 2 * N * S_f + P * N * (R_p + S_p)
-          + P * iters_patch * (2 * N + 2) * S_p + N * (2 * S_f + 2 * R_f))
-    b += N * S_f + nsum * S_f
-    return b
+          + P * iters_patch * (2 * N + 2) * S_p + N * (S_f + 2 * R_f))
+    if images == N:
+        return b + N * S_f + N * S_f + nsum * S_f
+    # the warp writes the node images and the plain sum
+    return b + (images + 1) * R_f + images * (R_f + S_f) + images * S_f + (nsum - 1) * S_f
 
 
 def measured_traffic(kernel):
@@ -324,12 +332,13 @@ def main():
     ms = (t1 - t0) * 1000.0 / (args.steps * K)
     g = L.geometry(W, H, 5, 5)
     # frame chunks per pass from the launches counted in the timed calls
-    per_launch = algorithmic_bytes(args.kernel, g, max(1, round(klaunch / (args.steps * K))))
+    images = SUM_IMAGES if res["frame_fmt_used"] == 0 else N
+    per_launch = algorithmic_bytes(args.kernel, g, max(1, round(klaunch / (args.steps * K))), images)
     avg_ms = kms / max(klaunch, 1)
     achieved = per_launch / (avg_ms * 1e-3) / 1e9 if klaunch else None
 
     gi, pi = iters[-1]
-    pb = path_bytes(g, gi, pi, ns)
+    pb = path_bytes(g, gi, pi, ns, images)
     # the FP64 oracle on the timed movie, before the optional legs below
     # reuse its device buffer
     cpu_leg = None
